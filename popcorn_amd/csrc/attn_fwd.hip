@@ -30,6 +30,8 @@
 // directly (no staging registers, no LDS stores), into buffers every wave
 // has finished with, and ends once they have landed; one barrier per step.
 // The head_dim-128 kernel fits three waves per SIMD (three blocks per CU).
+// Grids that cannot fill the CUs run wider blocks whose groups of 4 waves share
+// out the key tiles (NG below).
 //
 // Softmax with a fixed reference max: m is the row max of s * c over the
 // first key tile (key 0 is visible to every row) and stays put, so no step
@@ -77,7 +79,10 @@ namespace {
 using namespace attn;
 
 constexpr int BN = 32;
-constexpr int NT = 256;
+constexpr int NT = 256;  // threads of one key group (4 waves)
+constexpr int max_of(int a, int b) { return a > b ? a : b; }
+// Key groups of the split kernel: as many waves per SIMD as the rows' registers allow.
+template <int D> constexpr int kGroups = D <= 64 ? 4 : (D <= 128 ? 3 : 2);
 // fragment reads in flight ahead of the product that uses them (head_dim 256,
 // whose Q^T fragments and O^T accumulators take 192 registers, keeps fewer)
 template <int D> constexpr int kRing = D >= 192 ? 3 : (D == 32 ? 4 : 6);  // at most the step's 2 * D / 16 products
@@ -121,11 +126,17 @@ struct AttnArgs {
   int dr, dch;
 };
 
+// NG: key groups. One is the kernel described above. With more, the block is NG
+// times as wide, each group of 4 waves holds the same rows and heads and walks
+// every NG-th key tile through its own buffers, and the groups' O^T and l are
+// added through LDS at the end: what bounds a call of few blocks is the chain
+// of steps of its longest block at one wave per SIMD (0.54 us a step alone on a
+// CU at D 128; split, a CU takes three tiles in 1.2 us).
 // KS: 16-dim steps of the score products, D / 16, or one fewer when the row's
 // last 16 dims are all past head_dim (zeros in Q and K, so the step adds exact
 // zeros and skipping it changes no bit)
-template <typename T, int D, bool CAUSAL, int KS>
-__global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_eu(2))) void attn_fwd_kernel(
+template <typename T, int D, bool CAUSAL, int KS, int NG>
+__global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_waves_per_eu(2))) void attn_fwd_kernel(
     AttnArgs a) {
   using Frag = typename Mma<T>::frag;
   constexpr int KST = D + 8;   // K row stride in LDS, elements
@@ -133,8 +144,15 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   constexpr int KK = D / 16;
   constexpr int DT = D / 32;
   static_assert(KS == KK || KS == KK - 1, "at most the last 16-dim step is skipped");
-  __shared__ __attribute__((aligned(16))) T Ks[2][BN * KST];
-  __shared__ __attribute__((aligned(16))) T Vs[2][BN * D];
+  // Each key group's two K and two V tiles. With one group they are arrays of
+  // their own, which the compiler can tell apart; with several they share one
+  // area with the sums the groups hand over at the end.
+  constexpr int KT = BN * KST, VT = BN * D;
+  constexpr int kMerge = 4 * (DT * 16 + 1) * 64;  // floats one group hands over: O^T and l of four waves
+  constexpr int kArea = NG == 1 ? 16 : max_of(NG * 2 * (KT + VT) * (int)sizeof(T), (NG - 1) * kMerge * 4);
+  __shared__ __attribute__((aligned(16))) T Ks1[NG == 1 ? 2 * KT : 8];
+  __shared__ __attribute__((aligned(16))) T Vs1[NG == 1 ? 2 * VT : 8];
+  __shared__ __attribute__((aligned(16))) unsigned char area[kArea];
 
   // ---- work item: (q tile, batch, kv head, head quad) -- a group is one
   // (batch, kv head, quad). A block's waves are gp q heads of one kv group x
@@ -160,7 +178,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   const int b = rest / (a.Hkv * n_quads);
   const int hkv = (rest / n_quads) % a.Hkv;
   const int quad = rest % n_quads;
-  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // key group (NG > 1) and wave within it
+  const int kgrp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & (NG == 1 ? ~0 : 3);
   const int hq = hkv * G + quad * GP + wave_id % GP;
   const int rows_per_block = 32 * (4 / GP);
 
@@ -174,13 +194,22 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   const int m0 = m_tile * rows_per_block;
   if (m0 >= S) return;  // whole block: before any barrier
 
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = NG == 1 ? threadIdx.x : threadIdx.x & (NT - 1);
+  const int wave = NG == 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : wave_id;
   const int lane = tid & 63;
   const int r32 = lane & 31;
   const int g = lane >> 5;
   const int wave_first = m0 + (wave / GP) * 32;
   const int q_row = wave_first + r32;
+  auto kbuf_of = [&](int grp, int buf) -> T* {
+    if constexpr (NG == 1) return Ks1 + buf * KT;
+    else return reinterpret_cast<T*>(area) + grp * 2 * (KT + VT) + buf * KT;
+  };
+  auto kbuf = [&](int buf) { return kbuf_of(kgrp, buf); };
+  auto vbuf = [&](int buf) -> T* {
+    if constexpr (NG == 1) return Vs1 + buf * VT;
+    else return reinterpret_cast<T*>(area) + kgrp * 2 * (KT + VT) + 2 * KT + buf * VT;
+  };
 
   const T* qbase = static_cast<const T*>(a.q) + b * a.qsb + hq * a.qsh + start * a.qss;
   const T* kbase = static_cast<const T*>(a.k) + b * a.ksb + hkv * a.ksh + start * a.kss;
@@ -275,9 +304,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
       if (KSLOTS % NT == 0 || i * NT + tid < KSLOTS)
       {
         if constexpr (kAsmLoads)
-          ld_lds16_asm(kwords, Ks[buf] + (i * NT + wave * 64) * 8, kgo[i], tile);
+          ld_lds16_asm(kwords, kbuf(buf) + (i * NT + wave * 64) * 8, kgo[i], tile);
         else
-          ld_buf_lds(krsrc, Ks[buf] + (i * NT + wave * 64) * 8, kgo[i], tile);
+          ld_buf_lds(krsrc, kbuf(buf) + (i * NT + wave * 64) * 8, kgo[i], tile);
       }
   };
   auto dma_v = [&](int t, int buf) {
@@ -287,25 +316,24 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
       if constexpr (VWHOLE)
       {
         if constexpr (kAsmLoads)
-          ld_lds16_asm(vwords, Vs[buf] + (i * NT + wave * 64) * 8, vgo[0],
+          ld_lds16_asm(vwords, vbuf(buf) + (i * NT + wave * 64) * 8, vgo[0],
                        tile + i * (NT / KCH) * (int)a.vss * (int)sizeof(T));
         else
-          ld_buf_lds(vrsrc, Vs[buf] + (i * NT + wave * 64) * 8, vgo[0],
+          ld_buf_lds(vrsrc, vbuf(buf) + (i * NT + wave * 64) * 8, vgo[0],
                      tile + i * (NT / KCH) * (int)a.vss * (int)sizeof(T));
       }
       else if (VSLOTS % NT == 0 || i * NT + wave * 64 < VSLOTS)  // wave-uniform
       {
         if constexpr (kAsmLoads)
-          ld_lds16_asm(vwords, Vs[buf] + (i * NT + wave * 64) * 8, vgo[i], tile);
+          ld_lds16_asm(vwords, vbuf(buf) + (i * NT + wave * 64) * 8, vgo[i], tile);
         else
-          ld_buf_lds(vrsrc, Vs[buf] + (i * NT + wave * 64) * 8, vgo[i], tile);
+          ld_buf_lds(vrsrc, vbuf(buf) + (i * NT + wave * 64) * 8, vgo[i], tile);
       }
     }
   };
   auto landed = [&]() { lds_loads_landed(); };
   // S^T of the K tile in buffer buf
-  auto scores = [&](int buf) {
-    const T* ks = Ks[buf];
+  auto scores = [&](const T* ks) {
     f32x16 s;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = 0.f;
@@ -338,7 +366,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) acc[dt] = Mma<T>::run(vfrag(Vs[buf], c, dt), pf[c], acc[dt]);
+      for (int dt = 0; dt < DT; ++dt) acc[dt] = Mma<T>::run(vfrag(vbuf(buf), c, dt), pf[c], acc[dt]);
   };
   float m_i;  // reference max of s * c for query q_row
   float l_i;  // this lane's half of the denominator
@@ -365,13 +393,19 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
 
   // ---- fast sweep: fixed max; each step exponentiates S(t), then runs the
   // products of O += V(t)^T P(t)^T and S(t+1) over the same S registers
+  // Key group k of NG takes tiles k, k + NG, ...; all run the same number of
+  // steps, tiles past the end being masked whole (their V is the last tile's).
+  // Every group takes its reference max from tile 0, so their sums add up
+  // without rescaling.
+  const int n_steps = NG == 1 ? n_tiles : (n_tiles + NG - 1) / NG;
+  auto tile_of = [&](int j) { return NG == 1 ? j : kgrp + NG * j; };
   clear();
-  dma_k(0, 0);
-  dma_v(0, 0);
-  dma_k(1, 1);  // past the end this reads zeros or keys nobody uses
+  dma_k(NG == 1 ? 0 : min(tile_of(0), n_tiles), 0);
+  dma_v(NG == 1 ? 0 : min(tile_of(0), n_tiles - 1), 0);
+  dma_k(NG == 1 ? 1 : min(tile_of(1), n_tiles), 1);  // past the end this reads zeros or keys nobody uses
   landed();
   __syncthreads();
-  f32x16 sc = scores(0);
+  f32x16 sc = scores(kbuf_of(0, 0));
   if (need_mask(0)) apply_mask(0, sc);
   {
     float mx = -INFINITY;
@@ -379,6 +413,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[r]);
     m_i = fmaxf(mx, __shfl_xor(mx, 32, 64)) * a.c;
   }
+  if (NG > 1 && kgrp > 0) sc = scores(kbuf(0));
   __syncthreads();  // K(0) is read; the first step overwrites its buffer
   Frag pf[2];
   // Step t. Buffers: V(t) in Vs[t&1] and K(t+1) in Ks[(t+1)&1] are read;
@@ -391,13 +426,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   // LDS fragment address is a lane register plus an immediate.
   auto step = [&](int t, auto parity) {
     constexpr int P = decltype(parity)::value;
-    dma_k(min(t + 2, n_tiles), P);
-    dma_v(min(t + 1, n_tiles - 1), P ^ 1);
-    if (need_mask(t)) apply_mask(t, sc);
+    dma_k(min(tile_of(t + 2), n_tiles), P);
+    dma_v(min(tile_of(t + 1), n_tiles - 1), P ^ 1);
+    if (need_mask(tile_of(t))) apply_mask(tile_of(t), sc);
     softmax(sc, m_i, pf);
-    const T* ks = Ks[P ^ 1] + k_lane;
+    const T* ks = kbuf(P ^ 1) + k_lane;
+    const T* vs = vbuf(P);
     auto fetch = [&](int i) -> Frag {
-      if (i < KK) return vfrag(Vs[P], i / DT, i % DT);
+      if (i < KK) return vfrag(vs, i / DT, i % DT);
       return *reinterpret_cast<const Frag*>(ks + 16 * (i - KK));
     };
     constexpr int N = KK + KS;  // 2 * DT == KK products of V^T P^T, KS of S^T
@@ -425,18 +461,45 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   };
   for (int t = 0;;) {
     step(t, std::integral_constant<int, 0>{});
-    if (++t >= n_tiles) break;
+    if (++t >= n_steps) break;
     step(t, std::integral_constant<int, 1>{});
-    if (++t >= n_tiles) break;
+    if (++t >= n_steps) break;
+  }
+  if constexpr (NG > 1) {
+    // groups 1 .. NG - 1 leave O^T and l in LDS (the tiles are done with: the
+    // last step ended with a barrier); group 0 adds them in order
+    float* mine = reinterpret_cast<float*>(area) + wave * (DT * 16 + 1) * 64 + lane;
+    if (kgrp > 0) {
+      float* out = mine + (kgrp - 1) * kMerge;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) out[(dt * 16 + r) * 64] = acc[dt][r];
+      out[DT * 16 * 64] = l_i;
+    }
+    __syncthreads();
+    if (kgrp == 0) {
+#pragma unroll
+      for (int k = 0; k < NG - 1; ++k) {
+        const float* in = mine + k * kMerge;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[dt][r] += in[(dt * 16 + r) * 64];
+        l_i += in[DT * 16 * 64];
+      }
+    }
   }
 
   {
     const float l_tot = l_i + __shfl_xor(l_i, 32, 64);
-    const bool bad = !(l_tot <= kFastLimit<T>) || !(fabsf(m_i) < INFINITY);
+    const bool bad = (NG == 1 || kgrp == 0) &&  // group 0 holds the sums
+                     (!(l_tot <= kFastLimit<T>) || !(fabsf(m_i) < INFINITY));
     if (__syncthreads_or(bad)) {
       // ---- exact sweep: online max; O and l are rescaled only when the max
       // grows by more than 2^8 (exponents stay <= 8, and o = acc / l uses the
-      // same max in both)
+      // same max in both); with several key groups each sweeps all the keys,
+      // and group 0's result is the one kept
       clear();
       m_i = -INFINITY;
       dma_k(0, 0);
@@ -446,7 +509,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
       for (int u = 0; u < n_tiles; ++u) {
         dma_k(min(u + 1, n_tiles - 1), (u + 1) & 1);
         dma_v(min(u + 1, n_tiles - 1), (u + 1) & 1);
-        f32x16 s = scores(u & 1);
+        f32x16 s = scores(kbuf(u & 1));
         if (need_mask(u)) apply_mask(u, s);
         float mx = -INFINITY;
 #pragma unroll
@@ -471,6 +534,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   }
 
   // ---- epilogue
+  if (NG > 1 && kgrp > 0) return;
   const float l_tot = l_i + __shfl_xor(l_i, 32, 64);
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   if (q_row < S) {
@@ -492,14 +556,46 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   }
 }
 
+template <typename T, int D, int KS, int NG>
+int launch_groups(const AttnArgs& a, bool causal, hipStream_t s) {
+  const int64_t blocks = (int64_t)a.m_tiles * a.B * a.Hq / a.gp;
+  if (causal)
+    hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, KS, NG>), dim3(blocks), dim3(NG * NT), 0, s, a);
+  else
+    hipLaunchKernelGGL((attn_fwd_kernel<T, D, false, KS, NG>), dim3(blocks), dim3(NG * NT), 0, s, a);
+  return launched("pk_attn_fwd");
+}
+
+// Whether to split a block's keys over kGroups<D> key groups. The split block
+// has a CU to itself and walks its tiles kGroups times faster, but pays about
+// 5 us once (the wider block's start and the sum over the groups), and its
+// groups share every barrier. So it is for grids that cannot fill the CUs with
+// blocks of one group, and rows long enough to earn the cost back. Measured
+// (us, one group -> split; bf16):
+//   one block per CU:  D 128, 256 tiles causal 169 -> 103; 32 tiles full 24.7 -> 25.3;
+//                      D 64, 64 tiles causal 31.0 -> 22.8, 33 tiles full 17.8 -> 15.9
+//   two, causal:       D 128, 512 tiles 377 -> 265, 64 tiles 53.4 -> 50.2;
+//                      D 192, 128 tiles 130 -> 113; D 64, 64 tiles 35.3 -> 39.5
+//   two, full:         D 128, 64 tiles 66.9 -> 79.8 (the blocks are equally long and two share a CU)
+//   four:              D 128, 128 tiles causal 134 -> 155
+template <int D> bool split_keys(const AttnArgs& a, int64_t blocks, bool causal) {
+  const int tiles = (a.S + BN - 1) / BN;
+  // packed sequences: at most one partial q tile each beside the whole ones
+  if (a.cu != nullptr) {
+    const int64_t rows = 32 * (4 / a.gp);
+    const int64_t live = (a.total / rows + a.B) * (a.Hq / a.gp);
+    blocks = live < blocks ? live : blocks;
+  }
+  const int64_t cus = cu_count();
+  if (blocks <= cus) return tiles >= (D <= 64 ? 32 : 48);
+  return blocks <= 2 * cus && causal && tiles >= (D <= 64 ? 192 : 96);
+}
+
 template <typename T, int D, int KS>
 int launch_ks(const AttnArgs& a, bool causal, hipStream_t s) {
   const int64_t blocks = (int64_t)a.m_tiles * a.B * a.Hq / a.gp;
-  if (causal)
-    hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, KS>), dim3(blocks), dim3(NT), 0, s, a);
-  else
-    hipLaunchKernelGGL((attn_fwd_kernel<T, D, false, KS>), dim3(blocks), dim3(NT), 0, s, a);
-  return launched("pk_attn_fwd");
+  return split_keys<D>(a, blocks, causal) ? launch_groups<T, D, KS, kGroups<D>>(a, causal, s)
+                                          : launch_groups<T, D, KS, 1>(a, causal, s);
 }
 
 // head_dim 8-16, 40-48 and 72-80 (Popcorn's 16, 48 and 80) leave the last 16
