@@ -63,6 +63,17 @@ int pk_swiglu_bwd(const void* dy, const void* a, const void* b, void* da, void* 
                   void* stream);
 
 /*
+ * The same with a and b as `rows` rows of `cols` elements that lie a_stride and
+ * b_stride elements apart (the halves of one gate/up projection, say), read
+ * where they are. y, dy, da and db are contiguous [rows, cols] and overlap no
+ * input. Strides are not negative.
+ */
+int pk_swiglu_rows_fwd(const void* a, const void* b, void* y, int64_t rows, int64_t cols, int64_t a_stride,
+                       int64_t b_stride, int dtype, void* stream);
+int pk_swiglu_rows_bwd(const void* dy, const void* a, const void* b, void* da, void* db, int64_t rows, int64_t cols,
+                       int64_t a_stride, int64_t b_stride, int dtype, void* stream);
+
+/*
  * RMSNorm forward over `rows` contiguous rows of `cols` elements:
  *   r = 1/sqrt(mean(x^2) + eps); n = round_x(x*r); y = n * w [+ bias],
  * each product and sum rounded to w_dtype. x has `dtype`; w, bias and y have

@@ -32,6 +32,8 @@ SIGNATURES = {
     "pk_last_error": (ctypes.c_char_p, []),
     "pk_swiglu_fwd": (_int, [_p, _p, _p, _i64, _int, _p]),
     "pk_swiglu_bwd": (_int, [_p, _p, _p, _p, _p, _i64, _int, _p]),
+    "pk_swiglu_rows_fwd": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _int, _p]),
+    "pk_swiglu_rows_bwd": (_int, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p]),
     "pk_rmsnorm_fwd": (_int, [_p, _p, _p, _p, _p, _i64, _i64, _f32, _int, _int, _p]),
     "pk_rmsnorm_bwd_workspace": (_i64, [_i64, _i64, _int]),
     "pk_rmsnorm_bwd": (_int, [_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _int, _p]),

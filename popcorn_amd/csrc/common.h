@@ -57,6 +57,23 @@ template <typename T> __device__ __forceinline__ void st16_stream(T* p, const Ve
   __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(&r), reinterpret_cast<u32x4*>(p));
 }
 
+// The same sixteen bytes at any element's address: the hardware takes a 16-byte
+// access at a 2- or 4-byte boundary, the compiler has to be told of it.
+typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+template <bool ALIGNED, typename T> __device__ __forceinline__ Vec<T> ld16_stream_at(const T* p) {
+  if constexpr (ALIGNED) return ld16_stream(p);
+  Vec<T> r;
+  const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+  *reinterpret_cast<u32x4*>(&r) = v;
+  return r;
+}
+
+template <bool ALIGNED, typename T> __device__ __forceinline__ void st16_stream_at(T* p, const Vec<T>& r) {
+  if constexpr (ALIGNED) st16_stream(p, r);
+  else __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(&r), reinterpret_cast<u32x4_any*>(p));
+}
+
 // N elements of E whose bytes are a whole number of 16-byte vectors: the pack
 // of a wider type that lines up with one Vec of a narrower one (8 fp32 beside
 // 8 bf16 values, say), moved as one or more 16-byte accesses.

@@ -1,12 +1,18 @@
-// SwiGLU forward / backward: one HBM stream over n elements.
+// SwiGLU forward / backward: one HBM stream over rows x cols elements.
 //
 // Each thread moves one 16-byte vector of every operand, loads issued before
 // any arithmetic; data is touched once, so loads and stores are
 // non-temporal. Small blocks with one vector per thread measured fastest on
 // MI355X (forward 64 threads: 0.84 of the 8 TB/s spec at a, b [16384, 14336];
 // backward 128 threads), ahead of larger blocks or several vectors per
-// thread. A 1024-block grid-stride scalar launch finishes a ragged tail;
-// unaligned pointers take the scalar kernel for the whole range.
+// thread.
+//
+// a and b may be rows of a wider tensor (the halves of one gate/up projection):
+// each has a row stride, everything else is contiguous. Contiguous operands are
+// one row of all the elements, whose ragged end its last thread takes element
+// by element. In strided rows the last vector is the one that ends with the
+// row: where the width is ragged it overlaps the vector before it and writes
+// the same values there. Rows shorter than a vector take the scalar kernels.
 #include "api.h"
 #include "common.h"
 
@@ -16,7 +22,6 @@ namespace {
 constexpr int kThreads = 256;   // scalar kernels
 constexpr int kFwdThreads = 64;  // vector kernels: threads per block
 constexpr int kBwdThreads = 128;
-constexpr int kUnroll = 1;       // 16-byte vectors per operand per thread
 
 // sigmoid(a) in fp32 from the hardware exp2 and reciprocal (each ~1 ulp): the
 // stream is HBM-bound only while the per-element VALU work stays this short.
@@ -38,118 +43,192 @@ template <typename T> __device__ __forceinline__ void bwd_elem(T g, T a, T b, T&
   db = from_f32<T>(gf * af * s);
 }
 
-template <typename T>
+// A thread's vector of rows x cols elements: row r, starting at column c.
+struct Rows {
+  int64_t cols;
+  int64_t as, bs;       // row strides of a and b, elements
+  uint32_t nvec;        // vectors per row, the last one ending with the row
+  uint32_t mul, pre, shift;  // i / nvec = (((i - h) >> pre) + h) >> shift with h = mulhi(i, mul), for any 32-bit i
+};
+
+__device__ __forceinline__ void locate(const Rows& g, uint32_t i, int vec, int64_t& r, int64_t& c) {
+  const uint32_t h = __umulhi(i, g.mul);
+  const uint32_t q = (((i - h) >> g.pre) + h) >> g.shift;
+  r = q;
+  c = (int64_t)(i - q * g.nvec) * vec;
+  c = c + vec <= g.cols ? c : g.cols - vec;
+}
+
+template <typename T, bool ROWS, bool ALIGNED>
 __global__ __launch_bounds__(kFwdThreads) void swiglu_fwd_vec(const T* __restrict__ a, const T* __restrict__ b,
-                                                              T* __restrict__ y, int64_t nvec) {
+                                                              T* __restrict__ y, int64_t nvec, Rows g) {
   constexpr int P = Vec<T>::N;
-  constexpr int kThreads = kFwdThreads;
-  const int64_t base = (int64_t)blockIdx.x * (kThreads * kUnroll) + threadIdx.x;
-  Vec<T> va[kUnroll], vb[kUnroll];
-#pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    const int64_t i = base + (int64_t)u * kThreads;
-    if (i < nvec) {
-      va[u] = ld16_stream(a + i * P);
-      vb[u] = ld16_stream(b + i * P);
+  const int64_t i = (int64_t)blockIdx.x * kFwdThreads + threadIdx.x;
+  if (i >= nvec) return;
+  int64_t ao, bo, yo;
+  if constexpr (ROWS) {
+    int64_t r, c;
+    locate(g, (uint32_t)i, P, r, c);
+    ao = r * g.as + c;
+    bo = r * g.bs + c;
+    yo = r * g.cols + c;
+  } else {
+    ao = bo = yo = i * P;
+    if (ao + P > g.cols) {  // the ragged end: the last thread's alone
+      for (; ao < g.cols; ++ao) y[ao] = fwd_elem(a[ao], b[ao]);
+      return;
     }
   }
+  const Vec<T> va = ld16_stream_at<ALIGNED>(a + ao), vb = ld16_stream_at<ALIGNED>(b + bo);
+  Vec<T> vy;
 #pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    const int64_t i = base + (int64_t)u * kThreads;
-    if (i < nvec) {
-      Vec<T> vy;
-#pragma unroll
-      for (int j = 0; j < P; ++j) vy.v[j] = fwd_elem(va[u].v[j], vb[u].v[j]);
-      st16_stream(y + i * P, vy);
-    }
-  }
+  for (int j = 0; j < P; ++j) vy.v[j] = fwd_elem(va.v[j], vb.v[j]);
+  st16_stream_at<ALIGNED>(y + yo, vy);
 }
 
 template <typename T>
 __global__ __launch_bounds__(kThreads) void swiglu_fwd_scalar(const T* __restrict__ a, const T* __restrict__ b,
-                                                              T* __restrict__ y, int64_t start, int64_t n) {
-  for (int64_t i = start + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
-    y[i] = fwd_elem(a[i], b[i]);
+                                                              T* __restrict__ y, int64_t n, Rows g) {
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
+    const int64_t r = i / g.cols, c = i - r * g.cols;
+    y[i] = fwd_elem(a[r * g.as + c], b[r * g.bs + c]);
+  }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBwdThreads) void swiglu_bwd_vec(const T* __restrict__ g, const T* __restrict__ a,
+template <typename T, bool ROWS, bool ALIGNED>
+__global__ __launch_bounds__(kBwdThreads) void swiglu_bwd_vec(const T* __restrict__ dy, const T* __restrict__ a,
                                                               const T* __restrict__ b, T* __restrict__ da,
-                                                              T* __restrict__ db, int64_t nvec) {
+                                                              T* __restrict__ db, int64_t nvec, Rows g) {
   constexpr int P = Vec<T>::N;
-  constexpr int kThreads = kBwdThreads;
-  const int64_t base = (int64_t)blockIdx.x * (kThreads * kUnroll) + threadIdx.x;
-  Vec<T> vg[kUnroll], va[kUnroll], vb[kUnroll];
-#pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    const int64_t i = base + (int64_t)u * kThreads;
-    if (i < nvec) {
-      vg[u] = ld16_stream(g + i * P);
-      va[u] = ld16_stream(a + i * P);
-      vb[u] = ld16_stream(b + i * P);
+  const int64_t i = (int64_t)blockIdx.x * kBwdThreads + threadIdx.x;
+  if (i >= nvec) return;
+  int64_t ao, bo, yo;
+  if constexpr (ROWS) {
+    int64_t r, c;
+    locate(g, (uint32_t)i, P, r, c);
+    ao = r * g.as + c;
+    bo = r * g.bs + c;
+    yo = r * g.cols + c;
+  } else {
+    ao = bo = yo = i * P;
+    if (ao + P > g.cols) {  // the ragged end: the last thread's alone
+      for (; ao < g.cols; ++ao) bwd_elem(dy[ao], a[ao], b[ao], da[ao], db[ao]);
+      return;
     }
   }
+  const Vec<T> vg = ld16_stream_at<ALIGNED>(dy + yo);
+  const Vec<T> va = ld16_stream_at<ALIGNED>(a + ao), vb = ld16_stream_at<ALIGNED>(b + bo);
+  Vec<T> vda, vdb;
 #pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    const int64_t i = base + (int64_t)u * kThreads;
-    if (i < nvec) {
-      Vec<T> vda, vdb;
-#pragma unroll
-      for (int j = 0; j < P; ++j) bwd_elem(vg[u].v[j], va[u].v[j], vb[u].v[j], vda.v[j], vdb.v[j]);
-      st16_stream(da + i * P, vda);
-      st16_stream(db + i * P, vdb);
-    }
-  }
+  for (int j = 0; j < P; ++j) bwd_elem(vg.v[j], va.v[j], vb.v[j], vda.v[j], vdb.v[j]);
+  st16_stream_at<ALIGNED>(da + yo, vda);
+  st16_stream_at<ALIGNED>(db + yo, vdb);
 }
 
 template <typename T>
-__global__ __launch_bounds__(kThreads) void swiglu_bwd_scalar(const T* __restrict__ g, const T* __restrict__ a,
+__global__ __launch_bounds__(kThreads) void swiglu_bwd_scalar(const T* __restrict__ dy, const T* __restrict__ a,
                                                               const T* __restrict__ b, T* __restrict__ da,
-                                                              T* __restrict__ db, int64_t start, int64_t n) {
-  for (int64_t i = start + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
-    bwd_elem(g[i], a[i], b[i], da[i], db[i]);
+                                                              T* __restrict__ db, int64_t n, Rows g) {
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
+    const int64_t r = i / g.cols, c = i - r * g.cols;
+    bwd_elem(dy[i], a[r * g.as + c], b[r * g.bs + c], da[i], db[i]);
+  }
 }
 
 int64_t blocks_for(int64_t work, int64_t per_block) { return (work + per_block - 1) / per_block; }
 
-template <typename T> int fwd(const void* a, const void* b, void* y, int64_t n, hipStream_t stream) {
-  constexpr int P = Vec<T>::N;
-  const T* ap = static_cast<const T*>(a);
-  const T* bp = static_cast<const T*>(b);
-  T* yp = static_cast<T*>(y);
-  const bool vec = aligned16(a) && aligned16(b) && aligned16(y);
-  const int64_t nvec = vec ? n / P : 0;
-  if (nvec > 0)
-    hipLaunchKernelGGL(swiglu_fwd_vec<T>, dim3(blocks_for(nvec, kFwdThreads * kUnroll)), dim3(kFwdThreads), 0, stream,
-                       ap, bp, yp, nvec);
-  const int64_t rest = n - nvec * P;
-  if (rest > 0) {
-    const int64_t grid = blocks_for(rest, kThreads) < 1024 ? blocks_for(rest, kThreads) : 1024;
-    hipLaunchKernelGGL(swiglu_fwd_scalar<T>, dim3(grid), dim3(kThreads), 0, stream, ap, bp, yp, nvec * P, n);
-  }
-  return launched("pk_swiglu_fwd");
+// The tensors of a call: dy, da, db and y are contiguous [rows, cols].
+struct Call {
+  const void *dy, *a, *b;
+  void *y, *da, *db;
+};
+
+// Rows of the layout for the vector kernels: the multiplier of the exact 32-bit
+// division by nvec (Granlund and Montgomery's round-up method).
+template <int P> Rows rows_of(int64_t cols, int64_t as, int64_t bs) {
+  Rows g{cols, as, bs, (uint32_t)((cols + P - 1) / P), 0, 0, 0};
+  int l = 0;
+  while (l < 32 && ((uint64_t)1 << l) < g.nvec) ++l;  // ceil(log2(nvec))
+  g.mul = (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << l) - g.nvec)) / g.nvec + 1);
+  g.pre = l > 0 ? 1 : 0;
+  g.shift = l > 0 ? l - 1 : 0;
+  return g;
 }
 
-template <typename T>
-int bwd(const void* g, const void* a, const void* b, void* da, void* db, int64_t n, hipStream_t stream) {
+// Launches one slab of rows. Vectors are aligned when every row of every tensor
+// starts on 16 bytes and strided rows are whole vectors. Elsewhere they are
+// loaded and stored across 16-byte boundaries (bf16 forward, us: contiguous
+// [8192, 14336] 103.6, halves of one tensor 105.7 where copying the halves first
+// took 277; one operand 2 bytes off 108.9, by element it took the scalar
+// kernel; halves of an odd width, [8192, 14335], 128.3).
+template <typename T, bool BWD>
+void launch_slab(const Call& t, int64_t rows, int64_t cols, int64_t as, int64_t bs, hipStream_t s) {
   constexpr int P = Vec<T>::N;
-  const T* gp = static_cast<const T*>(g);
-  const T* ap = static_cast<const T*>(a);
-  const T* bp = static_cast<const T*>(b);
-  T* dap = static_cast<T*>(da);
-  T* dbp = static_cast<T*>(db);
-  const bool vec = aligned16(g) && aligned16(a) && aligned16(b) && aligned16(da) && aligned16(db);
-  const int64_t nvec = vec ? n / P : 0;
-  if (nvec > 0)
-    hipLaunchKernelGGL(swiglu_bwd_vec<T>, dim3(blocks_for(nvec, kBwdThreads * kUnroll)), dim3(kBwdThreads), 0,
-                       stream, gp, ap, bp, dap, dbp, nvec);
-  const int64_t rest = n - nvec * P;
-  if (rest > 0) {
-    const int64_t grid = blocks_for(rest, kThreads) < 1024 ? blocks_for(rest, kThreads) : 1024;
-    hipLaunchKernelGGL(swiglu_bwd_scalar<T>, dim3(grid), dim3(kThreads), 0, stream, gp, ap, bp, dap, dbp, nvec * P,
-                       n);
+  constexpr int NTB = BWD ? kBwdThreads : kFwdThreads;
+  const T *dy = static_cast<const T*>(t.dy), *a = static_cast<const T*>(t.a), *b = static_cast<const T*>(t.b);
+  T *y = static_cast<T*>(t.y), *da = static_cast<T*>(t.da), *db = static_cast<T*>(t.db);
+  if (cols < P && rows > 1) {
+    const Rows g{cols, as, bs, 0, 0, 0, 0};
+    const int64_t n = rows * cols, grid = blocks_for(n, kThreads) < 1024 ? blocks_for(n, kThreads) : 1024;
+    if constexpr (BWD)
+      hipLaunchKernelGGL(swiglu_bwd_scalar<T>, dim3(grid), dim3(kThreads), 0, s, dy, a, b, da, db, n, g);
+    else
+      hipLaunchKernelGGL(swiglu_fwd_scalar<T>, dim3(grid), dim3(kThreads), 0, s, a, b, y, n, g);
+    return;
   }
-  return launched("pk_swiglu_bwd");
+  const Rows g = rows_of<P>(cols, as, bs);
+  const int64_t per_row = (cols + P - 1) / P, nvec = rows * per_row;
+  bool aligned = aligned16(a) && aligned16(b);
+  if (rows > 1) aligned = aligned && cols % P == 0 && as % P == 0 && bs % P == 0;
+  aligned = aligned && (BWD ? aligned16(dy) && aligned16(da) && aligned16(db) : aligned16(y));
+  const dim3 grid((unsigned)blocks_for(nvec, NTB)), block(NTB);
+#define PK_SWIGLU(ROWS, ALIGNED)                                                                               \
+  if constexpr (BWD)                                                                                           \
+    hipLaunchKernelGGL((swiglu_bwd_vec<T, ROWS, ALIGNED>), grid, block, 0, s, dy, a, b, da, db, nvec, g);      \
+  else                                                                                                         \
+    hipLaunchKernelGGL((swiglu_fwd_vec<T, ROWS, ALIGNED>), grid, block, 0, s, a, b, y, nvec, g);
+  if (rows == 1) {
+    if (aligned) { PK_SWIGLU(false, true) } else { PK_SWIGLU(false, false) }
+  } else {
+    if (aligned) { PK_SWIGLU(true, true) } else { PK_SWIGLU(true, false) }
+  }
+#undef PK_SWIGLU
+}
+
+template <typename T, bool BWD>
+int run(const char* who, Call t, int64_t rows, int64_t cols, int64_t as, int64_t bs, hipStream_t s) {
+  if (rows > 1 && as == cols && bs == cols) {  // contiguous: one row
+    cols *= rows;
+    rows = 1;
+  }
+  // slabs of rows whose vectors have 32-bit indexes (one row has 64-bit ones)
+  const int64_t per_row = (cols + Vec<T>::N - 1) / Vec<T>::N;
+  int64_t most = INT32_MAX / per_row;
+  most = rows == 1 || most < 1 ? 1 : most;
+  const auto at = [](const void* p, int64_t n) { return const_cast<void*>(static_cast<const void*>(static_cast<const T*>(p) + n)); };
+  for (int64_t r = 0; r < rows; r += most) {
+    const int64_t n = rows - r < most ? rows - r : most;
+    const Call c = BWD ? Call{at(t.dy, r * cols), at(t.a, r * as), at(t.b, r * bs), nullptr, at(t.da, r * cols), at(t.db, r * cols)}
+                       : Call{nullptr, at(t.a, r * as), at(t.b, r * bs), at(t.y, r * cols), nullptr, nullptr};
+    launch_slab<T, BWD>(c, n, cols, as, bs, s);
+  }
+  return launched(who);
+}
+
+template <bool BWD>
+int dispatch(const char* who, const Call& t, int64_t rows, int64_t cols, int64_t as, int64_t bs, int dtype, void* stream) {
+  if (rows < 0 || cols < 0)
+    return fail(PK_ERR_INVALID, "%s: negative size (%lld, %lld)", who, (long long)rows, (long long)cols);
+  if (rows == 0 || cols == 0) return PK_OK;
+  if (!t.a || !t.b || (BWD ? !t.dy || !t.da || !t.db : !t.y)) return fail(PK_ERR_INVALID, "%s: null pointer", who);
+  if (as < 0 || bs < 0) return fail(PK_ERR_INVALID, "%s: negative row stride", who);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (dtype) {
+    case PK_F32: return run<float, BWD>(who, t, rows, cols, as, bs, s);
+    case PK_BF16: return run<bf16, BWD>(who, t, rows, cols, as, bs, s);
+    case PK_F16: return run<f16, BWD>(who, t, rows, cols, as, bs, s);
+  }
+  return fail(PK_ERR_UNSUPPORTED, "%s: dtype code %d", who, dtype);
 }
 
 }  // namespace
@@ -158,32 +237,24 @@ int bwd(const void* g, const void* a, const void* b, void* da, void* db, int64_t
 extern "C" {
 
 int pk_swiglu_fwd(const void* a, const void* b, void* y, int64_t n, int dtype, void* stream) {
-  using namespace pk;
-  if (n < 0) return fail(PK_ERR_INVALID, "pk_swiglu_fwd: negative size %lld", (long long)n);
-  if (n == 0) return PK_OK;
-  if (!a || !b || !y) return fail(PK_ERR_INVALID, "pk_swiglu_fwd: null pointer");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (dtype) {
-    case PK_F32: return fwd<float>(a, b, y, n, s);
-    case PK_BF16: return fwd<bf16>(a, b, y, n, s);
-    case PK_F16: return fwd<f16>(a, b, y, n, s);
-  }
-  return fail(PK_ERR_UNSUPPORTED, "pk_swiglu_fwd: dtype code %d", dtype);
+  return pk::dispatch<false>("pk_swiglu_fwd", {nullptr, a, b, y, nullptr, nullptr}, 1, n, 0, 0, dtype, stream);
 }
 
 int pk_swiglu_bwd(const void* dy, const void* a, const void* b, void* da, void* db, int64_t n, int dtype,
                   void* stream) {
-  using namespace pk;
-  if (n < 0) return fail(PK_ERR_INVALID, "pk_swiglu_bwd: negative size %lld", (long long)n);
-  if (n == 0) return PK_OK;
-  if (!dy || !a || !b || !da || !db) return fail(PK_ERR_INVALID, "pk_swiglu_bwd: null pointer");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (dtype) {
-    case PK_F32: return bwd<float>(dy, a, b, da, db, n, s);
-    case PK_BF16: return bwd<bf16>(dy, a, b, da, db, n, s);
-    case PK_F16: return bwd<f16>(dy, a, b, da, db, n, s);
-  }
-  return fail(PK_ERR_UNSUPPORTED, "pk_swiglu_bwd: dtype code %d", dtype);
+  return pk::dispatch<true>("pk_swiglu_bwd", {dy, a, b, nullptr, da, db}, 1, n, 0, 0, dtype, stream);
+}
+
+int pk_swiglu_rows_fwd(const void* a, const void* b, void* y, int64_t rows, int64_t cols, int64_t a_stride,
+                       int64_t b_stride, int dtype, void* stream) {
+  return pk::dispatch<false>("pk_swiglu_rows_fwd", {nullptr, a, b, y, nullptr, nullptr}, rows, cols, a_stride, b_stride,
+                             dtype, stream);
+}
+
+int pk_swiglu_rows_bwd(const void* dy, const void* a, const void* b, void* da, void* db, int64_t rows, int64_t cols,
+                       int64_t a_stride, int64_t b_stride, int dtype, void* stream) {
+  return pk::dispatch<true>("pk_swiglu_rows_bwd", {dy, a, b, nullptr, da, db}, rows, cols, a_stride, b_stride, dtype,
+                            stream);
 }
 
 }  // extern "C"

@@ -276,44 +276,76 @@ def add_rms_norm(x: Tensor, residual: Tensor, weight: Tensor, eps: float = 1e-6,
 # --------------------------------------------------------------------------- swiglu
 
 
-def _swiglu_fwd(a: Tensor, b: Tensor) -> tuple[Tensor, Tensor, Tensor]:
-    """One pk_swiglu_fwd launch: (y, a and b as the contiguous tensors it read)."""
+def _row_stride(t: Tensor) -> int | None:
+    """Elements between consecutive rows (of the last dimension) when one stride says where every row of t
+    starts, as for the halves of a fused projection; None when it does not."""
+    if t.dim() < 2 or t.stride(-1) != 1 or t.numel() == 0 or t.is_neg():
+        return None
+    stride, span = None, 1  # the innermost leading dimension's stride, and how many of it lie within
+    for size, step in zip(reversed(t.shape[:-1]), reversed(t.stride()[:-1])):
+        if size == 1:
+            continue
+        if stride is None:
+            stride = step
+        elif step != stride * span:
+            return None
+        span *= size
+    return t.shape[-1] if stride is None else stride
+
+
+def _swiglu_operands(a: Tensor, b: Tensor) -> tuple[Tensor, Tensor, int, int]:
+    """a and b as the kernels read them, and their row strides: in place wherever rows have one, else copied."""
+    if not (a.is_contiguous() and b.is_contiguous()):
+        strides = _row_stride(a), _row_stride(b)
+        if None not in strides:
+            return a, b, *strides
+    cols = a.shape[-1] if a.dim() else 1
+    return a.contiguous(), b.contiguous(), cols, cols
+
+
+def _swiglu_fwd(a: Tensor, b: Tensor) -> tuple[Tensor, tuple[Tensor, Tensor, int, int]]:
+    """One launch: (y, a and b as it read them with their row strides)."""
     device = _require_cuda(a, b)
     dtype = _same_dtype("swiglu", a, b)
     if a.shape != b.shape:
         raise ValueError(f"popcorn_amd.swiglu: shapes differ {tuple(a.shape)} vs {tuple(b.shape)}")
-    a_c, b_c = a.contiguous(), b.contiguous()
-    y = torch.empty_like(a_c)
+    operands = a_r, b_r, a_stride, b_stride = _swiglu_operands(a, b)
+    y = torch.empty(a.shape, dtype=dtype, device=device)
+    cols = a.shape[-1] if a.dim() else 1
+    rows = a.numel() // cols if cols else 0
     lib = _lib.load()
     with _lib.on_device(device):
         _lib.check(
-            lib.pk_swiglu_fwd(
-                a_c.data_ptr(), b_c.data_ptr(), y.data_ptr(), a_c.numel(), _lib.dtype_code(dtype),
+            lib.pk_swiglu_rows_fwd(
+                a_r.data_ptr(), b_r.data_ptr(), y.data_ptr(), rows, cols, a_stride, b_stride, _lib.dtype_code(dtype),
                 _lib.stream_handle(device),
             ),
             lib,
         )
-    return y, a_c, b_c
+    return y, operands
 
 
 class _SwiGLU(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a: Tensor, b: Tensor) -> Tensor:
-        y, a_c, b_c = _swiglu_fwd(a, b)
-        ctx.save_for_backward(a_c, b_c)
+        y, (a_r, b_r, *ctx.strides) = _swiglu_fwd(a, b)
+        ctx.save_for_backward(a_r, b_r)
         return y
 
     @staticmethod
     def backward(ctx, dy: Tensor):
-        a_c, b_c = ctx.saved_tensors
-        g = dy.to(a_c.dtype).contiguous()
-        da, db = torch.empty_like(a_c), torch.empty_like(b_c)
+        a, b = ctx.saved_tensors
+        g = dy.to(a.dtype).contiguous()
+        da = torch.empty(a.shape, dtype=a.dtype, device=a.device)
+        db = torch.empty(b.shape, dtype=b.dtype, device=b.device)
+        cols = a.shape[-1] if a.dim() else 1
+        rows = a.numel() // cols if cols else 0
         lib = _lib.load()
-        with _lib.on_device(a_c.device):
+        with _lib.on_device(a.device):
             _lib.check(
-                lib.pk_swiglu_bwd(
-                    g.data_ptr(), a_c.data_ptr(), b_c.data_ptr(), da.data_ptr(), db.data_ptr(), a_c.numel(),
-                    _lib.dtype_code(a_c.dtype), _lib.stream_handle(a_c.device),
+                lib.pk_swiglu_rows_bwd(
+                    g.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(), db.data_ptr(), rows, cols, *ctx.strides,
+                    _lib.dtype_code(a.dtype), _lib.stream_handle(a.device),
                 ),
                 lib,
             )
