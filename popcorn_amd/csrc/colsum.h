@@ -1,7 +1,5 @@
-// Deterministic column sums of a [parts, cols] fp32 array of per-block partial
-// rows (weight gradients), in a fixed order so repeated runs give identical
-// bits. Stage one: block (cx, s) sums parts [s*kColSplit, (s+1)*kColSplit) of
-// 256 columns into stage[s]; stage two sums the stage rows and rounds to T.
+// Deterministic column sums of [parts, cols] fp32 arrays of per-block partial
+// rows (weight gradients), in a fixed order so repeated runs give identical bits.
 #pragma once
 
 #include "common.h"
@@ -9,71 +7,75 @@
 namespace pk {
 namespace {
 
-constexpr int kColThreads = 256;
-constexpr int kColSplit = 32;  // partial rows summed per block in the first stage
+// out[c] = sum over p of part[p * cols + c], rounded once to the output's type.
+struct ColumnSum {
+  const float* part;
+  void* out;
+  int64_t parts;
+};
 
-// v[p0 * ld] + ... + v[(p1 - 1) * ld], added in index order; loads are issued
-// eight at a time so their latencies overlap.
-__device__ __forceinline__ float ordered_sum(const float* __restrict__ v, int64_t ld, int64_t p0, int64_t p1) {
+// A block takes kColCols columns with kColLanes row lanes each: lane l adds rows
+// l, l + kColLanes, ... 16 at a time, as a tree, and the lanes are then added as
+// trees too, in an order that depends on nothing but `parts`. What bounds it is
+// the latency of a lane's chain of loads (the partial rows are in the L2 or the
+// MALL), so the lanes are many and the columns few, 16 columns still being whole
+// 64-byte pieces of a row: 1280 x 4096 partial rows take 5.0 us, in one launch,
+// where a stage per 32 rows and a final one took 5.1 + 3.9, and the two sums of
+// 2048 x 1537 (dw and dbias) 11.2 where they took 19.
+constexpr int kColCols = 16;
+constexpr int kColLanes = 64;
+constexpr int kColThreads = kColCols * kColLanes;
+constexpr int kColWaves = kColThreads / 64;
+
+// t[0] + ... + t[N - 1] as a tree (overwrites t)
+template <int N> __device__ __forceinline__ float tree_sum(float (&t)[N]) {
+#pragma unroll
+  for (int w = N / 2; w >= 1; w /= 2)
+#pragma unroll
+    for (int u = 0; u < w; ++u) t[u] += t[u + w];
+  return t[0];
+}
+
+// Two sums of one width in one launch (dw and dbias, or the q and the k weight): blockIdx.y picks.
+template <typename T>
+__global__ __launch_bounds__(kColThreads) void column_sum(ColumnSum first, ColumnSum second, int cols) {
+  __shared__ float acc[kColWaves][kColCols];
+  const ColumnSum j = blockIdx.y == 0 ? first : second;
+  const int cl = threadIdx.x % kColCols, rl = threadIdx.x / kColCols;
+  const int c = blockIdx.x * kColCols + cl;
   float s = 0.f;
-  int64_t p = p0;
-  for (; p + 8 <= p1; p += 8) {
-    float t[8];
+  if (c < cols) {
+    const float* v = j.part + c;
+    const int64_t step = (int64_t)kColLanes * cols;
+    int64_t p = rl;
+    for (; p + 15 * kColLanes < j.parts; p += 16 * kColLanes) {
+      float t[16];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) t[u] = v[(p + u) * ld];
+      for (int u = 0; u < 16; ++u) t[u] = v[p * cols + u * step];
+      s += tree_sum(t);
+    }
+    float t[16];  // the lane's last rows, all in flight together
 #pragma unroll
-    for (int u = 0; u < 8; ++u) s += t[u];
+    for (int u = 0; u < 16; ++u) t[u] = p + u * kColLanes < j.parts ? v[p * cols + u * step] : 0.f;
+    s += tree_sum(t);
   }
-  for (; p < p1; ++p) s += v[p * ld];
-  return s;
+  // the wave's four row lanes of each column, then the waves
+  s += __shfl_xor(s, 16, 64);
+  s += __shfl_xor(s, 32, 64);
+  if (threadIdx.x % 64 < kColCols) acc[threadIdx.x / 64][cl] = s;
+  __syncthreads();
+  if (threadIdx.x < kColCols && c < cols) {
+    float t[kColWaves];
+#pragma unroll
+    for (int w = 0; w < kColWaves; ++w) t[w] = acc[w][cl];
+    static_cast<T*>(j.out)[c] = from_f32<T>(tree_sum(t));
+  }
 }
-
-__global__ __launch_bounds__(kColThreads) void column_sum_stage(const float* __restrict__ part,
-                                                               float* __restrict__ stage, int64_t parts, int cols) {
-  const int c = blockIdx.x * kColThreads + threadIdx.x;
-  const int64_t p0 = (int64_t)blockIdx.y * kColSplit;
-  const int64_t p1 = p0 + kColSplit < parts ? p0 + kColSplit : parts;
-  if (c >= cols) return;
-  stage[(int64_t)blockIdx.y * cols + c] = ordered_sum(part + c, cols, p0, p1);
-}
-
-// A block takes kFinalCols columns with kFinalLanes row lanes each: lane l sums
-// stage rows l, l + kFinalLanes, ... in order, then lane 0 adds the lanes in
-// order, so the result is the same on every run.
-constexpr int kFinalCols = 32;
-constexpr int kFinalLanes = kColThreads / kFinalCols;
 
 template <typename T>
-__global__ __launch_bounds__(kColThreads) void column_sum_final(const float* __restrict__ stage, T* __restrict__ out,
-                                                               int64_t n, int cols) {
-  __shared__ float acc[kFinalLanes][kFinalCols];
-  const int cl = threadIdx.x % kFinalCols, rl = threadIdx.x / kFinalCols;
-  const int c = blockIdx.x * kFinalCols + cl;
-  float s = 0.f;
-  if (c < cols && rl < n) s = ordered_sum(stage + rl * (int64_t)cols + c, (int64_t)kFinalLanes * cols, 0,
-                                          (n - rl + kFinalLanes - 1) / kFinalLanes);
-  acc[rl][cl] = s;
-  __syncthreads();
-  if (rl == 0 && c < cols) {
-    float t = acc[0][cl];
-#pragma unroll
-    for (int r = 1; r < kFinalLanes; ++r) t += acc[r][cl];
-    out[c] = from_f32<T>(t);
-  }
-}
-
-// Rows of the first-stage array for `parts` partial rows.
-inline int64_t stage_rows(int64_t parts) { return (parts + kColSplit - 1) / kColSplit; }
-
-// out[c] = sum over p of part[p * cols + c], rounded once to T; stage holds
-// stage_rows(parts) * cols floats.
-template <typename T> void column_sums(const float* part, float* stage, T* out, int64_t parts, int cols,
-                                       hipStream_t s) {
-  const int64_t n = stage_rows(parts);
-  const int cx = (cols + kColThreads - 1) / kColThreads;
-  hipLaunchKernelGGL(column_sum_stage, dim3(cx, (unsigned)n), dim3(kColThreads), 0, s, part, stage, parts, cols);
-  hipLaunchKernelGGL(column_sum_final<T>, dim3((cols + kFinalCols - 1) / kFinalCols), dim3(kColThreads), 0, s, stage,
-                     out, n, cols);
+void column_sums(const ColumnSum& first, const ColumnSum* second, int cols, hipStream_t s) {
+  hipLaunchKernelGGL(column_sum<T>, dim3((cols + kColCols - 1) / kColCols, second ? 2 : 1), dim3(kColThreads), 0, s,
+                     first, second ? *second : first, cols);
 }
 
 }  // namespace

@@ -21,8 +21,8 @@
 // block) with w and its running dw / dbias columns in registers, prefetching
 // the next row's x and dy while the current row's dot product is reduced.
 // Blocks leave one fp32 partial row each (the rows of a block's wavefront
-// slots are combined through LDS first), and a two-stage column reduction
-// sums the partials in a fixed order, so dw is deterministic.
+// slots are combined through LDS first), and a column reduction sums the
+// partials in a fixed order, so dw is deterministic.
 //
 // Types: T is x's type (and dx's); W is the weight's, which is also the type
 // of the bias, of y and of dy, and of dw / dbias: W = T, or fp32 with a 16-bit
@@ -585,7 +585,7 @@ struct BwdArgs {
   float offset;
   const float* rstd;
   void *dx, *dw, *db;
-  float *dw_part, *db_part, *stage;
+  float *dw_part, *db_part;
   int64_t rows;
   int cols;
   hipStream_t s;
@@ -663,15 +663,14 @@ template <typename T, typename W, int MODE> int bwd(const BwdArgs& a, const char
                        static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.rstd, static_cast<const W*>(a.dy),
                        static_cast<const T*>(a.ds), a.offset, static_cast<T*>(a.dx), a.dw_part, a.db_part, a.rows,
                        a.cols, 1.0f / (float)a.cols);
-  column_sums<W>(a.dw_part, a.stage, static_cast<W*>(a.dw), blocks, a.cols, a.s);
-  if (MODE == kBias) column_sums<W>(a.db_part, a.stage, static_cast<W*>(a.db), blocks, a.cols, a.s);
+  const ColumnSum db{a.db_part, a.db, blocks};
+  column_sums<W>({a.dw_part, a.dw, blocks}, MODE == kBias ? &db : nullptr, a.cols, a.s);
   return launched(who);
 }
 
-// Workspace: [blocks, cols] dw partials, the same for dbias, and the
-// [stage_rows, cols] first-stage column sums, each rounded up to 256 bytes.
+// Workspace: [blocks, cols] dw partials and the same for dbias, each rounded up to 256 bytes.
 struct Layout {
-  int64_t part, stage, total;
+  int64_t part, total;
 };
 
 template <typename T, typename W, int MODE> Layout layout_for(int64_t rows, int64_t cols) {
@@ -682,8 +681,7 @@ template <typename T, typename W, int MODE> Layout layout_for(int64_t rows, int6
   auto up = [](int64_t n) { return (n + 255) / 256 * 256; };
   Layout l;
   l.part = up(blocks * cols * (int64_t)sizeof(float));
-  l.stage = up(stage_rows(blocks) * cols * (int64_t)sizeof(float));
-  l.total = l.part * (MODE == kBias ? 2 : 1) + l.stage;
+  l.total = l.part * (MODE == kBias ? 2 : 1);
   return l;
 }
 
@@ -752,7 +750,6 @@ int carve(const char* who, void* workspace, int64_t workspace_bytes, int64_t row
   char* base = static_cast<char*>(workspace);
   a.dw_part = reinterpret_cast<float*>(base);
   a.db_part = mode == kBias ? reinterpret_cast<float*>(base + l.part) : nullptr;
-  a.stage = reinterpret_cast<float*>(base + l.part * (mode == kBias ? 2 : 1));
   return PK_OK;
 }
 
@@ -771,13 +768,11 @@ int check_shape(const char* who, int64_t rows, int64_t cols, int dtype, int wdty
 }  // namespace pk
 
 // ---------------------------------------------------------------------------
-// Fixed scratch for pk_rmsnorm_bwd_noalloc: the dw / dbias partial rows and
-// the column-sum stage of one backward call. Every GPU the library runs on
-// holds its own copy from module load until the process ends. Each block
-// writes its whole partial row and the first column-sum stage writes every
-// stage row it covers, so nothing needs clearing between calls; two calls that
-// overlap on one GPU (on different streams, or from different threads) share
-// the array and race.
+// Fixed scratch for pk_rmsnorm_bwd_noalloc: the dw / dbias partial rows of one
+// backward call. Every GPU the library runs on holds its own copy from module
+// load until the process ends. Each block writes its whole partial row, so
+// nothing needs clearing between calls; two calls that overlap on one GPU (on
+// different streams, or from different threads) share the array and race.
 static constexpr int64_t kScratchBytes = (int64_t)96 << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -842,7 +837,7 @@ int pk_rmsnorm_bwd(const void* x, const void* w, const float* rstd, const void* 
     return fail(PK_ERR_INVALID, "pk_rmsnorm_bwd: null pointer");
   if (rows == 0) return fail(PK_ERR_UNSUPPORTED, "pk_rmsnorm_bwd: zero rows (dw is all zeros; fill it host-side)");
   const int mode = dbias != nullptr ? kBias : kPlain;
-  BwdArgs a{x, w, dy, nullptr, 0.f, rstd, dx, dw, dbias, nullptr, nullptr, nullptr, rows, (int)cols,
+  BwdArgs a{x, w, dy, nullptr, 0.f, rstd, dx, dw, dbias, nullptr, nullptr, rows, (int)cols,
             static_cast<hipStream_t>(stream)};
   if (int st = carve(who, workspace, workspace_bytes, rows, cols, dtype, w_dtype, mode, a)) return st;
   return mode == kBias ? bwd_dispatch<kBias>(a, dtype, w_dtype, who) : bwd_dispatch<kPlain>(a, dtype, w_dtype, who);
@@ -866,7 +861,7 @@ int pk_rmsnorm_bwd_noalloc(const void* x, const void* w, const float* rstd, cons
   if (!x || !w || !rstd || !dy || !dx || !dw) return fail(PK_ERR_INVALID, "%s: null pointer", who);
   void* base = nullptr;
   if (int st = scratch_address(who, &base)) return st;
-  BwdArgs a{x, w, dy, nullptr, 0.f, rstd, dx, dw, dbias, nullptr, nullptr, nullptr, rows, (int)cols,
+  BwdArgs a{x, w, dy, nullptr, 0.f, rstd, dx, dw, dbias, nullptr, nullptr, rows, (int)cols,
             static_cast<hipStream_t>(stream)};
   if (int st = carve(who, base, kScratchBytes, rows, cols, dtype, w_dtype, mode, a)) return st;
   return mode == kBias ? bwd_dispatch<kBias>(a, dtype, w_dtype, who) : bwd_dispatch<kPlain>(a, dtype, w_dtype, who);
@@ -896,7 +891,7 @@ int pk_add_rmsnorm_bwd(const void* s, const void* w, const float* rstd, const vo
     return fail(PK_ERR_INVALID, "pk_add_rmsnorm_bwd: null pointer");
   if (rows == 0) return fail(PK_ERR_UNSUPPORTED, "pk_add_rmsnorm_bwd: zero rows (dw is all zeros; fill it host-side)");
   if (!isfinite(offset)) return fail(PK_ERR_INVALID, "pk_add_rmsnorm_bwd: offset is not finite");
-  BwdArgs a{s, w, dy, ds, offset, rstd, dx, dw, nullptr, nullptr, nullptr, nullptr, rows, (int)cols,
+  BwdArgs a{s, w, dy, ds, offset, rstd, dx, dw, nullptr, nullptr, nullptr, rows, (int)cols,
             static_cast<hipStream_t>(stream)};
   if (int st = carve(who, workspace, workspace_bytes, rows, cols, dtype, w_dtype, kAdd, a)) return st;
   return bwd_dispatch<kAdd>(a, dtype, w_dtype, who);

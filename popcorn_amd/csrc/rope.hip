@@ -235,8 +235,8 @@ int run_types(int in_dtype, int out_dtype, int cs_dtype, bool vec, const void* c
 // are butterflies over them. A head group never mixes q and k heads, so a
 // block holds one weight vector and one dw accumulator. dw is reduced without
 // atomics: lanes of one chunk column in a wave, then the four waves through
-// LDS, into one [2 * head_dim] partial row per block (the other side's half
-// zero), summed over blocks in a fixed order by column_sums.
+// LDS, into one [head_dim] partial row per block (q's blocks first, then k's),
+// summed over a side's blocks in a fixed order by column_sums.
 
 struct NormArgs {
   const void* x[2];   // q, k
@@ -252,7 +252,7 @@ struct NormArgs {
   int group[2];       // heads per block of q and of k
   int groups_q;       // head groups of q; groups [groups_q, groups_q + groups_k) are k's
   float eps, inv_d;
-  float* part;        // backward: [blocks, 2 * head_dim] partial dw rows
+  float* part;        // backward: [blocks, head_dim] partial dw rows, q's blocks first
 };
 
 struct NormPlan {
@@ -456,13 +456,8 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_bwd_kernel(const C* __r
     }
   }
   __syncthreads();
-  float* out = a.part + (int64_t)blockIdx.x * 2 * hd;
-  for (int c = threadIdx.x; c < 2 * hd; c += kThreads) {
-    const int side = c >= hd, col = c - side * hd;
-    float v = 0.f;
-    if (side == t) v = ((red[col] + red[hd + col]) + red[2 * hd + col]) + red[3 * hd + col];
-    out[c] = v;
-  }
+  float* out = a.part + (int64_t)blockIdx.x * hd;
+  for (int c = threadIdx.x; c < hd; c += kThreads) out[c] = ((red[c] + red[hd + c]) + red[2 * hd + c]) + red[3 * hd + c];
 }
 
 // 16-byte chunks with a power-of-two count per row, at most 64; 0 when unsupported.
@@ -475,9 +470,7 @@ int norm_chunks(int64_t head_dim, int x_dtype) {
 }
 
 int64_t norm_workspace(const NormPlan& p, int64_t head_dim) {
-  auto up = [](int64_t n) { return (n + 255) / 256 * 256; };
-  const int64_t cols = 2 * head_dim;
-  return up(p.blocks * cols * (int64_t)sizeof(float)) + up(stage_rows(p.blocks) * cols * (int64_t)sizeof(float));
+  return (p.blocks * head_dim * (int64_t)sizeof(float) + 255) / 256 * 256;
 }
 
 // TY: the forward's output type, which is the backward's cotangent type; W: the weights' type
@@ -493,19 +486,17 @@ int norm_launch(bool backward, const void* cs, const void* sn, NormArgs a, const
                          c, n, a);
     return launched("pk_qk_norm_rope_fwd");
   }
-  const int cols = 4 * a.half;
-  auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
+  const int hd = 2 * a.half;
   a.part = static_cast<float*>(ws);
-  float* stage = reinterpret_cast<float*>(static_cast<char*>(ws) + up(p.blocks * cols * (int64_t)sizeof(float)));
   if (p.blocks > 0) {
-    const size_t lds = 4 * (size_t)(2 * a.half) * sizeof(float);
+    const size_t lds = 4 * (size_t)hd * sizeof(float);
     hipLaunchKernelGGL((qk_norm_rope_bwd_kernel<T, TY, C, W, VEC, 2>), dim3((unsigned)p.blocks), dim3(kThreads), lds,
                        s, c, n, a);
-    column_sums<W>(a.part, stage, static_cast<W*>(dw), p.blocks, cols, s);
-  } else {  // nothing to sum: dw is zero
-    hipLaunchKernelGGL(column_sum_final<W>, dim3((cols + kFinalCols - 1) / kFinalCols), dim3(kColThreads), 0, s,
-                       stage, static_cast<W*>(dw), (int64_t)0, cols);
   }
+  // a side without blocks sums nothing: its dw is zero
+  const int64_t q_blocks = (int64_t)a.batch * p.tiles * p.groups_q;
+  const ColumnSum k_sum{a.part + q_blocks * hd, static_cast<W*>(dw) + hd, p.blocks - q_blocks};
+  column_sums<W>({a.part, dw, q_blocks}, &k_sum, hd, s);
   return launched("pk_qk_norm_rope_bwd");
 }
 
