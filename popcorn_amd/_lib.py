@@ -9,6 +9,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -88,6 +89,45 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         if path is None:
             _lib = lib
         return lib
+
+
+NATIVE = LIBRARY.with_name("_native.so")
+
+
+class _ThroughPython:
+    """Stands for the native call path where it cannot be used: every call is declined."""
+
+    def __getattr__(self, name):
+        return lambda *args: NotImplemented
+
+
+_native = None
+
+
+def native():
+    """The native call path (`csrc/host.cpp`): the same calls into the library without Python and ctypes.
+
+    It is an extension module of the torch it was built against. Where that is not the running one, or it
+    has not been built, calls go through Python, several times slower on the host, with a warning.
+    """
+    global _native
+    if _native is not None:
+        return _native
+    if not LIBRARY.exists():  # the call itself says so, after its other checks
+        return _ThroughPython()
+    load()
+    try:
+        from popcorn_amd import _native as module
+
+        if module.ABI_VERSION != ABI_VERSION or module.TORCH_VERSION != torch.__version__:
+            raise ImportError(f"built for ABI {module.ABI_VERSION} and torch {module.TORCH_VERSION}")
+        module.set_error(KernelError)
+        _native = module
+    except ImportError as e:
+        warnings.warn(f"popcorn_amd: {NATIVE.name} cannot be used ({e}); calls go through Python. Rebuild with "
+                      "`python -m popcorn_amd.build`", RuntimeWarning, stacklevel=3)
+        _native = _ThroughPython()
+    return _native
 
 
 def check(status: int, lib: ctypes.CDLL | None = None) -> None:

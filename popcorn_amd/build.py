@@ -1,8 +1,10 @@
 """Build recipe for the HIP kernel library: hipcc for gfx950, in-tree output.
 
 `python -m popcorn_amd.build` compiles every `csrc/*.hip` to an object in
-`popcorn_amd/_build/` (in parallel) and links `popcorn_amd/libpopcorn_amd.so`.
-The library is always rebuilt: the call is the "does it build" check. Asked
+`popcorn_amd/_build/` (in parallel) and links `popcorn_amd/libpopcorn_amd.so`,
+and `csrc/host.cpp`, the calls into it that do not pass through Python, to
+`popcorn_amd/_native.so`, an extension module of the running Python and torch.
+Both are always rebuilt: the call is the "does it build" check. Asked
 to (`python -m popcorn_amd.build` and `__graft_entry__.build()` ask), it then
 writes the `popcorn-amd` distribution metadata beside the package in a source
 tree (setup.py's `egg_info`, as an editable install would), so Popcorn's
@@ -16,6 +18,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -23,6 +26,7 @@ PACKAGE = Path(__file__).resolve().parent
 CSRC = PACKAGE / "csrc"
 BUILD = PACKAGE / "_build"
 LIBRARY = PACKAGE / "libpopcorn_amd.so"
+NATIVE = PACKAGE / "_native.so"
 INCLUDE = PACKAGE.parent / "include"
 
 ARCH = "gfx950"
@@ -63,25 +67,51 @@ def _compile(source: Path) -> Path:
     return obj
 
 
+def _compile_host() -> Path:
+    """The extension module's object: host code only, against torch's and Python's headers."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    obj = BUILD / "host.o"
+    cmd = [hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+           f'-DPK_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *(f"-isystem{p}" for p in (*include_paths("cuda"), sysconfig.get_paths()["include"])),
+           "-c", str(CSRC / "host.cpp"), "-o", str(obj)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"hipcc failed on host.cpp:\n{proc.stderr}")
+    return obj
+
+
+def _link(output: Path, *args: str) -> None:
+    tmp = output.with_suffix(".so.tmp")
+    proc = subprocess.run([hipcc(), "-shared", "-fPIC", *args, "-o", str(tmp)], capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"link of {output.name} failed:\n{proc.stderr}")
+    os.replace(tmp, output)
+
+
 def build(verbose: bool = False, write_metadata: bool = False) -> Path:
-    """Compile all kernels and link the shared library; returns its path.
+    """Compile all kernels and the host calls and link both libraries; returns the kernels' path.
 
     With `write_metadata`, also write the distribution metadata into the source tree (see
     `write_source_metadata`).
     """
     BUILD.mkdir(exist_ok=True)
     srcs = sources()
-    workers = min(len(srcs), int(os.environ.get("MAX_JOBS", "8")), 16) or 1
+    workers = min(len(srcs) + 1, int(os.environ.get("MAX_JOBS", "8")), 16) or 1
     with ThreadPoolExecutor(max_workers=workers) as pool:
+        host = pool.submit(_compile_host)
         objects = list(pool.map(_compile, srcs))
-    tmp = LIBRARY.with_suffix(".so.tmp")
-    cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"link failed:\n{proc.stderr}")
-    os.replace(tmp, LIBRARY)
+        host = host.result()
+    _link(LIBRARY, f"--offload-arch={ARCH}", *map(str, objects))
+    import torch
+
+    # libpopcorn_amd.so is found beside the module; torch's libraries are loaded before it by `import torch`
+    _link(NATIVE, str(host), f"-L{PACKAGE}", f"-l:{LIBRARY.name}", "-Wl,-rpath,$ORIGIN",
+          f"-L{Path(torch.__file__).parent / 'lib'}", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip")
     if verbose:
-        print(f"built {LIBRARY} from {len(srcs)} sources", file=sys.stderr)
+        print(f"built {LIBRARY} from {len(srcs)} sources, and {NATIVE.name}", file=sys.stderr)
     if write_metadata:
         write_source_metadata()
     return LIBRARY

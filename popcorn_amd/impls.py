@@ -7,6 +7,11 @@ reference's output structure. Arithmetic happens in the HIP kernels of
 `libpopcorn_amd.so`, launched on torch's current stream; there is no
 host-side or torch fallback: an input the kernels do not cover raises.
 
+Each function first offers the call to the native path (`_lib.native`), which
+takes plain tensors in layouts the kernels read in place. What it declines
+(tensor subclasses, calls that are being traced or transformed, layouts that
+need a copy, empty tensors, and whatever has to be refused) is done here.
+
     rms_norm(x, weight, bias=None, eps=1e-6)        kernels/rms_norm.py:16-30
     add_rms_norm(x, residual, weight, eps=1e-6, offset=0.0)  kernels/add_rms_norm.py:8-26
     swiglu(a, b)                                    kernels/swiglu.py:9-18
@@ -25,6 +30,8 @@ import torch
 from torch import Tensor
 
 from popcorn_amd import _lib
+
+_compiling = torch.compiler.is_compiling  # a traced call stays in Python, where the tracer can follow it
 
 __all__ = ["rms_norm", "add_rms_norm", "swiglu", "rotary_embedding", "attn", "attn_with_lse", "attn_varlen",
            "attn_varlen_with_lse", "rotary_embedding_", "rope",
@@ -178,6 +185,10 @@ def rms_norm(x: Tensor, weight: Tensor, bias: Tensor | None = None, eps: float =
     (the weight's). Without a gradient to track, the call is one launch with no
     autograd node and no saved statistics.
     """
+    if not _compiling():
+        y = _lib.native().rms_norm(x, weight, bias, eps)
+        if y is not NotImplemented:
+            return y
     if _tracks_grad(x, weight, bias):
         return _RMSNorm.apply(x, weight, bias, eps)
     return _rms_norm_fwd(x, weight, bias, eps, want_rstd=False)[0]
@@ -267,6 +278,10 @@ def add_rms_norm(x: Tensor, residual: Tensor, weight: Tensor, eps: float = 1e-6,
     (kernels/add_rms_norm.py:26). Backward gives d(x) = d(residual) in x's dtype
     and dweight in the weight's.
     """
+    if not _compiling():
+        ys = _lib.native().add_rms_norm(x, residual, weight, eps, offset)
+        if ys is not NotImplemented:
+            return ys
     if _tracks_grad(x, residual, weight):
         return _AddRMSNorm.apply(x, residual, weight, eps, offset)
     y, s, _, _ = _add_rms_norm_fwd(x, residual, weight, eps, offset)
@@ -328,13 +343,13 @@ def _swiglu_fwd(a: Tensor, b: Tensor) -> tuple[Tensor, tuple[Tensor, Tensor, int
 class _SwiGLU(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a: Tensor, b: Tensor) -> Tensor:
-        y, (a_r, b_r, *ctx.strides) = _swiglu_fwd(a, b)
+        y, (a_r, b_r, _, _) = _swiglu_fwd(a, b)
         ctx.save_for_backward(a_r, b_r)
         return y
 
     @staticmethod
     def backward(ctx, dy: Tensor):
-        a, b = ctx.saved_tensors
+        a, b, *strides = _swiglu_operands(*ctx.saved_tensors)  # a hook may hand them back in another layout
         g = dy.to(a.dtype).contiguous()
         da = torch.empty(a.shape, dtype=a.dtype, device=a.device)
         db = torch.empty(b.shape, dtype=b.dtype, device=b.device)
@@ -344,7 +359,7 @@ class _SwiGLU(torch.autograd.Function):
         with _lib.on_device(a.device):
             _lib.check(
                 lib.pk_swiglu_rows_bwd(
-                    g.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(), db.data_ptr(), rows, cols, *ctx.strides,
+                    g.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(), db.data_ptr(), rows, cols, *strides,
                     _lib.dtype_code(a.dtype), _lib.stream_handle(a.device),
                 ),
                 lib,
@@ -354,6 +369,10 @@ class _SwiGLU(torch.autograd.Function):
 
 def swiglu(a: Tensor, b: Tensor) -> Tensor:
     """y = silu(a) * b elementwise (a, b of one shape and dtype); differentiable."""
+    if not _compiling():
+        y = _lib.native().swiglu(a, b)
+        if y is not NotImplemented:
+            return y
     if _tracks_grad(a, b):
         return _SwiGLU.apply(a, b)
     return _swiglu_fwd(a, b)[0]
@@ -435,6 +454,10 @@ def rotary_embedding(x: Tensor, cos: Tensor, sin: Tensor, interleaved: bool = Fa
     NeoX halves by default, GPT-J pairs with interleaved=True; channels past
     2*half are passed through. Returns a new tensor; cos and sin get no gradient.
     """
+    if not _compiling():
+        y = _lib.native().rotary_embedding(x, cos, sin, interleaved)
+        if y is not NotImplemented:
+            return y
     if _tracks_grad(x):
         return _Rotary.apply(x, cos, sin, interleaved)
     return _rotary_fwd(x, cos, sin, interleaved)[0]
@@ -523,6 +546,10 @@ def rope(q: Tensor, k: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor
     row may differ. fp32 arithmetic, one rounding per output; one launch for q
     and k. Gradients have q/k's dtype; cos and sin get none.
     """
+    if not _compiling():
+        ys = _lib.native().rope(q, k, cos, sin)
+        if ys is not NotImplemented:
+            return ys
     if _tracks_grad(q, k):
         return _Rope.apply(q, k, cos, sin)
     return _rope(q, k, cos, sin, transpose=False)
@@ -633,6 +660,10 @@ def qk_norm_rope(q: Tensor, k: Tensor, q_weight: Tensor, k_weight: Tensor, cos: 
     Backward gives dq, dk in q's dtype and the two weight gradients in the
     weights'; cos and sin get none.
     """
+    if not _compiling():
+        ys = _lib.native().qk_norm_rope(q, k, q_weight, k_weight, cos, sin, eps)
+        if ys is not NotImplemented:
+            return ys
     if _tracks_grad(q, k, q_weight, k_weight):
         return _QkNormRope.apply(q, k, q_weight, k_weight, cos, sin, eps)
     return _qk_norm_rope_fwd(q, k, q_weight, k_weight, cos, sin, eps)[:2]
@@ -655,6 +686,10 @@ def attn(q: Tensor, k: Tensor, v: Tensor, causal: bool = False, softmax_scale: f
     bf16, fp16 or fp32 with head_dim a multiple of 8 up to 256; scale
     defaults to head_dim ** -0.5. Backward gives dq, dk, dv.
     """
+    if not _compiling():
+        o = _lib.native().attn(q, k, v, causal, softmax_scale)
+        if o is not NotImplemented:
+            return o
     if _tracks_grad(q, k, v):
         _grad_supported("attn", q.shape[-1], q.dtype)
         return _Attention.apply(q, k, v, causal, softmax_scale)
@@ -762,6 +797,10 @@ def attn_varlen(
     as for `attn`. Backward gives dq, dk, dv.
     """
     cu, num_seqs, longest = _cut_points(cu_seqlens, q.shape[0], q.device)
+    if not _compiling():
+        o = _lib.native().attn_varlen(q, k, v, cu, num_seqs, longest, causal, softmax_scale)
+        if o is not NotImplemented:
+            return o
     if _tracks_grad(q, k, v):
         _grad_supported("attn_varlen", q.shape[-1], q.dtype)
         return _AttentionVarlen.apply(q, k, v, cu, num_seqs, longest, causal, softmax_scale)

@@ -28,10 +28,10 @@ class BuildWithKernels(build_py):
     """Compile the HIP kernel library (hipcc, gfx950) before the package files are collected."""
 
     def run(self) -> None:
-        library = ROOT / "popcorn_amd" / "libpopcorn_amd.so"
         if os.environ.get("POPCORN_AMD_PREBUILT"):
-            if not library.exists():
-                raise SystemExit(f"POPCORN_AMD_PREBUILT is set but {library} has not been built")
+            for library in (ROOT / "popcorn_amd" / name for name in ("libpopcorn_amd.so", "_native.so")):
+                if not library.exists():
+                    raise SystemExit(f"POPCORN_AMD_PREBUILT is set but {library} has not been built")
         else:
             sys.path.insert(0, str(ROOT))
             from popcorn_amd import build
@@ -46,7 +46,7 @@ setup(
     description="MI355X (gfx950) HIP kernel backend for Popcorn's transformer-block ops",
     python_requires=">=3.10",
     packages=["popcorn_amd", "popcorn_amd.compat"],
-    package_data={"popcorn_amd": ["libpopcorn_amd.so", "csrc/*.hip", "csrc/*.h"]},
+    package_data={"popcorn_amd": ["libpopcorn_amd.so", "_native.so", "csrc/*.hip", "csrc/*.h", "csrc/*.cpp"]},
     install_requires=["torch", "numpy", "packaging", "pyarrow"],
     cmdclass={"build_py": BuildWithKernels},
     zip_safe=False,
