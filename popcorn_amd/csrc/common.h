@@ -105,6 +105,39 @@ template <typename E, int N> __device__ __forceinline__ void st_lane_stream(E* p
     __builtin_nontemporal_store(reinterpret_cast<const u32x4*>(r.v)[i], reinterpret_cast<u32x4*>(p) + i);
 }
 
+// The same packs at any element's address (see u32x4_any).
+template <bool ALIGNED, typename E, int N> __device__ __forceinline__ Lane<E, N> ld_lane_at(const E* p) {
+  if constexpr (ALIGNED) return ld_lane<E, N>(p);
+  Lane<E, N> r;
+#pragma unroll
+  for (int i = 0; i < Lane<E, N>::kVectors; ++i) reinterpret_cast<u32x4*>(r.v)[i] = reinterpret_cast<const u32x4_any*>(p)[i];
+  return r;
+}
+
+template <bool ALIGNED, typename E, int N> __device__ __forceinline__ void st_lane_at(E* p, const Lane<E, N>& r) {
+#pragma unroll
+  for (int i = 0; i < Lane<E, N>::kVectors; ++i) {
+    if constexpr (ALIGNED) reinterpret_cast<uint4*>(p)[i] = reinterpret_cast<const uint4*>(r.v)[i];
+    else reinterpret_cast<u32x4_any*>(p)[i] = reinterpret_cast<const u32x4*>(r.v)[i];
+  }
+}
+
+template <bool ALIGNED, typename E, int N> __device__ __forceinline__ Lane<E, N> ld_lane_stream_at(const E* p) {
+  if constexpr (ALIGNED) return ld_lane_stream<E, N>(p);
+  Lane<E, N> r;
+#pragma unroll
+  for (int i = 0; i < Lane<E, N>::kVectors; ++i)
+    reinterpret_cast<u32x4*>(r.v)[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p) + i);
+  return r;
+}
+
+template <bool ALIGNED, typename E, int N> __device__ __forceinline__ void st_lane_stream_at(E* p, const Lane<E, N>& r) {
+  if constexpr (ALIGNED) return st_lane_stream(p, r);
+#pragma unroll
+  for (int i = 0; i < Lane<E, N>::kVectors; ++i)
+    __builtin_nontemporal_store(reinterpret_cast<const u32x4*>(r.v)[i], reinterpret_cast<u32x4_any*>(p) + i);
+}
+
 // Sum over the 64 lanes of a wavefront; every lane receives the total.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
