@@ -95,6 +95,7 @@ struct BwdArgs {
   int nsplit;
   int64_t rows;
   int B, S, Hq, Hkv, group;
+  int live_q, live_k;  // packed sequences: q and key tiles per group that the grids hold (packed_item), or 0
   float scale;  // signed softmax scale
   float c;      // |scale| * log2(e), at least 1e-30
   uint32_t q_flip;
@@ -175,20 +176,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   const int rows_per_block = 32 * (4 / GP);
   const int m_tiles = (a.S + rows_per_block - 1) / rows_per_block;
   const int n_quads = G / GP;
-  const int per_tile = a.B * a.Hkv * n_quads;
   const int w = blockIdx.x;
-  int m_tile, rest;
-  if (per_tile % 8 == 0) {  // group-major per XCD, as in the forward
-    const int k = w >> 3;
-    m_tile = m_tiles - 1 - k % m_tiles;
-    rest = (w & 7) + 8 * (k / m_tiles);
-  } else {
-    m_tile = m_tiles - 1 - w / per_tile;
-    rest = w % per_tile;
-  }
-  const int b = rest / (a.Hkv * n_quads);
-  const int hkv = (rest / n_quads) % a.Hkv;
-  const int hq = hkv * G + (rest % n_quads) * GP + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % GP;
+  const WorkItem item =
+      a.live_q > 0 ? packed_item<CAUSAL>(w, a.cu, a.B, a.total, a.S, rows_per_block, a.Hkv * n_quads)
+                   : dense_item<CAUSAL>(w, a.B * a.Hkv * n_quads, a.Hkv * n_quads, m_tiles, a.S % rows_per_block != 0);
+  if (item.seq < 0) return;  // whole block, before any barrier
+  const int m_tile = item.tile, b = item.seq;
+  const int hkv = item.group / n_quads;
+  const int hq = hkv * G + (item.group % n_quads) * GP + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % GP;
   int start, S;
   seq_bounds(a, b, start, S);
   const int m0 = m_tile * rows_per_block;
@@ -410,6 +405,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
     finish();
   };
   static_assert(NSQ == 4, "the step loop is unrolled over four stage phases");
+  if (wave_first >= S) {  // a wave without rows: only its share of the loads
+    for (int t = 1; t <= n_tiles; ++t) {
+      issue(min(t + NSQ - 2, n_tiles - 1), (t + NSQ - 2) % NSQ);
+      finish();
+    }
+    lds_loads_landed();
+    return;  // past the block's last barrier
+  }
   for (int t = 1;;) {
     step(t, std::integral_constant<int, 1>{});
     if (++t > n_tiles) break;
@@ -469,17 +472,25 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   __shared__ __attribute__((aligned(16))) _Float16 Pb[2][4][16 * 64];
 
-  const int w = blockIdx.x;
-  const int per_tile = a.B * a.Hkv * a.nsplit;
   // first key tiles (the most causal work) first. (Group-major order per XCD,
-  // as the forward and dq kernels use, measured 26 % more HBM fetch here: a
-  // block streams its group's whole Q/dO from its own key tile on, and the
-  // 32 resident blocks of one group start at 32 different places.)
-  const int kv_tile = w / per_tile;
-  const int gi = w % per_tile;
-  const int b = gi / (a.Hkv * a.nsplit);
-  const int hkv = (gi / a.nsplit) % a.Hkv;
-  const int split = gi % a.nsplit;
+  // as the forward and dq kernels use for dense batches, measured 26 % more HBM
+  // fetch here: a block streams its group's whole Q/dO from its own key tile on,
+  // and the 32 resident blocks of one group start at 32 different places.)
+  int kv_tile, b, group;
+  if (a.live_k > 0) {
+    const WorkItem item = packed_item<false>(blockIdx.x, a.cu, a.B, a.total, a.S, BK, a.Hkv * a.nsplit);
+    if (item.seq < 0) return;  // whole block, before any barrier
+    kv_tile = item.tile;
+    b = item.seq;
+    group = item.group;
+  } else {
+    const int per_tile = a.B * a.Hkv * a.nsplit;
+    kv_tile = blockIdx.x / per_tile;
+    b = blockIdx.x % per_tile / (a.Hkv * a.nsplit);
+    group = blockIdx.x % (a.Hkv * a.nsplit);
+  }
+  const int hkv = group / a.nsplit;
+  const int split = group % a.nsplit;
   const int heads = a.group / a.nsplit;  // q heads this block walks, from split * heads on
   int start, S;
   seq_bounds(a, b, start, S);
@@ -742,6 +753,15 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   };
   using std::integral_constant;
   int t = 0;
+  if (kw0 >= S) {  // a slice without keys: only its waves' share of the loads
+    for (; t <= n_it + 1; ++t) {
+      issue((t + NS - 3) % NS);
+      loads_landed_but<(NS - 4) * PER_ISSUE>();
+      __syncthreads();
+    }
+    loads_landed_but<0>();
+    return;  // past the block's last barrier
+  }
   for (; t <= role; ++t) body(t, integral_constant<int, 0>{}, integral_constant<int, 0>{});  // tau <= 0
   static_assert(NS == 6, "the step loop is unrolled over six stage phases");
   for (;;) {  // tau = t - role >= 1, phase tau % NS = 1, 2, ..., 5, 0
@@ -823,14 +843,21 @@ __global__ __launch_bounds__(256) void dkdv_sum_kernel(BwdArgs a) {
   }
 }
 
+// The 16-bit dq kernel's grid; sets which of its work mappings applies.
+int64_t dq_grid(BwdArgs& a) {
+  const int gp = a.group % 4 == 0 ? 4 : (a.group % 2 == 0 ? 2 : 1), rows = 32 * (4 / gp);
+  a.live_q = packed_tiles(a.cu != nullptr, a.B, a.total, a.S, rows);
+  return (a.live_q > 0 ? a.live_q : (int64_t)((a.S + rows - 1) / rows) * a.B) * (a.Hq / gp);
+}
+
 #include "attn_bwd_f32.h"
 #include "attn_bwd_wide.h"
 
 template <typename T, int D, int KS>
-int launch_ks(const BwdArgs& a, bool causal, hipStream_t s) {
-  const int gp = a.group % 4 == 0 ? 4 : (a.group % 2 == 0 ? 2 : 1);
-  const int64_t dq_blocks = (int64_t)((a.S + 32 * (4 / gp) - 1) / (32 * (4 / gp))) * a.B * a.Hq / gp;
-  const int64_t kv_blocks = (int64_t)((a.S + BK - 1) / BK) * a.B * a.Hkv * a.nsplit;
+int launch_ks(BwdArgs a, bool causal, hipStream_t s) {
+  const int64_t dq_blocks = dq_grid(a);
+  a.live_k = packed_tiles(a.cu != nullptr, a.B, a.total, a.S, BK);
+  const int64_t kv_blocks = (a.live_k > 0 ? a.live_k : (int64_t)((a.S + BK - 1) / BK) * a.B) * a.Hkv * a.nsplit;
   if (causal) {
     hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, KS>), dim3(dq_blocks), dim3(NT), 0, s, a);
     hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, true, KS>), dim3(kv_blocks), dim3(NT2), 0, s, a);

@@ -263,9 +263,8 @@ void attn_bwd_dkdv_wide_kernel(BwdArgs a) {
 }
 
 // head_dim 136-256 in bf16 or fp16 (rows of D = 192 or 256): the dq kernel at D and the single-role dk/dv kernel
-template <typename T, int D> int launch_wide(const BwdArgs& a, bool causal, hipStream_t s) {
-  const int gp = a.group % 4 == 0 ? 4 : (a.group % 2 == 0 ? 2 : 1);
-  const int64_t dq_blocks = (int64_t)((a.S + 32 * (4 / gp) - 1) / (32 * (4 / gp))) * a.B * a.Hq / gp;
+template <typename T, int D> int launch_wide(BwdArgs a, bool causal, hipStream_t s) {
+  const int64_t dq_blocks = dq_grid(a);
   const int64_t kv_blocks = (int64_t)((a.S + BK - 1) / BK) * a.B * a.Hkv * a.nsplit;
   if (causal) {
     hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true>), dim3(dq_blocks), dim3(NT), 0, s, a);

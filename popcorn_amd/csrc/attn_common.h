@@ -49,6 +49,87 @@ __device__ __forceinline__ void ld_buf_lds4(__amdgpu_buffer_rsrc_t r, void* lds,
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 4, voffset, soffset, 0, 0);
 }
 
+// ---- which tile of rows (or keys) block w works on
+//
+// A "group" is what shares K/V: a (sequence, kv head, quad of q heads), say; a
+// sequence's `per_seq` groups are consecutive. Dispatch is round-robin over the
+// 8 XCDs, block w running on XCD w % 8.
+struct WorkItem {
+  int seq, group, tile;  // seq < 0: no work
+};
+
+// Dense batches, `groups` = sequences * per_seq of `tiles` tiles each, the last
+// of them partial if `partial`. With a multiple of 8 groups, XCD x runs groups
+// x, x + 8, ... one after another, so the blocks resident on an XCD share one
+// group's K/V in its L2; otherwise the tiles run one after another over all
+// groups. DESC (causal rows): the last tiles are the longest and go first.
+// Otherwise all tiles are alike but the partial ones, which go last, where a
+// short block fills what the whole ones leave (1025 rows of 12 heads of 64, a
+// batch of 8: the 96 blocks of one row each took slots of a first round that
+// the 768 whole blocks fill).
+template <bool DESC> __device__ __forceinline__ WorkItem dense_item(int w, int groups, int per_seq, int tiles, bool partial) {
+  int tile, rest;
+  if (!DESC && partial && tiles > 1 && w >= (tiles - 1) * groups) {
+    tile = tiles - 1;
+    rest = w - tile * groups;
+  } else {
+    if (!DESC && partial && tiles > 1) --tiles;
+    if (groups % 8 == 0) {
+      const int k = w >> 3;
+      tile = k % tiles;
+      rest = (w & 7) + 8 * (k / tiles);
+    } else {
+      tile = w / groups;
+      rest = w % groups;
+    }
+    if (DESC) tile = tiles - 1 - tile;
+  }
+  return {rest / per_seq, rest % per_seq, tile};
+}
+
+// Packed sequences, at most 64 of them: only the tiles that exist, the longest
+// sequence first (the blocks that run last are then short), all of a sequence's
+// tiles of one group on one XCD where per_seq is a multiple of 8. A grid of the
+// longest sequence's tiles for every sequence was three quarters empty blocks at
+// 23 documents of 44 to 3048 tokens, and ended with whatever came last. Each wave
+// finds its item alone: lane i holds sequence i's tiles and counts those of the
+// sequences in front of it.
+template <bool DESC>
+__device__ __forceinline__ WorkItem packed_item(int w, const int* cu, int seqs, int total, int longest, int rows, int per_seq) {
+  int u, group;
+  if (per_seq % 8 == 0) {
+    const int k = w >> 3, each = per_seq >> 3;
+    u = k / each;
+    group = (w & 7) + 8 * (k % each);
+  } else {
+    u = w / per_seq;
+    group = w % per_seq;
+  }
+  const int lane = threadIdx.x & 63;
+  int mine = 0;
+  if (lane < seqs) {
+    const int start = min(max(cu[lane], 0), total);
+    const int len = min(min(max(cu[lane + 1], start), total) - start, longest);
+    mine = (len + rows - 1) / rows;
+  }
+  int before = 0;
+  for (int j = 0; j < seqs; ++j) {
+    const int t = __builtin_amdgcn_readlane(mine, j);
+    before += t > mine || (t == mine && j < lane) ? t : 0;
+  }
+  const uint64_t found = __ballot(u >= before && u < before + mine);
+  if (found == 0) return {-1, 0, 0};
+  const int seq = __builtin_ctzll(found);
+  const int tile = u - __builtin_amdgcn_readlane(before, seq);
+  return {seq, group, DESC ? __builtin_amdgcn_readlane(mine, seq) - 1 - tile : tile};
+}
+
+// Tiles of `rows` that the packed sequences can have at most, when blocks are
+// to be found by packed_item; 0 when every sequence gets the longest one's.
+inline int packed_tiles(bool packed, int64_t seqs, int64_t total, int64_t longest, int64_t rows) {
+  return packed && seqs > 1 && seqs <= 64 && longest > rows ? (int)(total / rows + seqs) : 0;
+}
+
 // A buffer resource as its four words (base, 32-bit range, raw-buffer flags),
 // made wave-uniform, for the inline-assembly loads below.
 typedef unsigned rsrc_words __attribute__((ext_vector_type(4)));

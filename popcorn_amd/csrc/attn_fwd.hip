@@ -62,10 +62,9 @@
 //
 // K and V are read through buffer resources based at the (batch, kv head):
 // a tile is one scalar offset, and rows at or past S read as zero, so no load
-// is predicated; such keys are masked like causal ones. Work order: each XCD
-// (dispatch is round-robin over the 8 XCDs) runs its (batch, kv head) groups
-// one after another, longest causal rows first within a group, so the blocks
-// resident on an XCD read the same K/V prefix.
+// is predicated; such keys are masked like causal ones. Work order: dense_item
+// and packed_item (attn_common.h); at the shape above, each XCD running its
+// groups one after another takes 4.4x less HBM fetch than interleaving four.
 #include <math.h>
 
 #include <type_traits>
@@ -118,6 +117,7 @@ struct AttnArgs {
   int64_t qsb, qss, qsh, ksb, kss, ksh, vsb, vss, vsh, osb, oss, osh;
   int64_t lse_bs, lse_hs;  // lse element (b, h, token t of b) at b*lse_bs + h*lse_hs + t (+ cu[b] when packed)
   int B, S, Hq, Hkv, group, m_tiles;
+  int live;  // packed sequences: q tiles per group of heads that the grid holds (packed_item), or 0
   int gp;  // q heads of one kv group per block (4, 2 or 1); the block's 4 waves are gp heads x 4/gp row groups
   float c;          // |scale| * log2(e), at least 1e-30
   uint32_t q_flip;  // 0x80008000 when scale < 0 (negates both halves of a packed pair), else 0
@@ -161,28 +161,17 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
   const int n_quads = G / GP;
   const int per_tile = a.B * a.Hkv * n_quads;
   const int w = blockIdx.x;
-  // With a multiple of 8 groups, XCD x (block w runs on XCD w % 8) takes
-  // groups x, x + 8, ... one after another, each group's q tiles longest
-  // first: the ~96 blocks resident on an XCD then share one group's K/V
-  // prefix in its L2 (4.4x less HBM fetch at C5 than interleaving four
-  // groups per XCD). Otherwise q tiles run longest first over all groups.
-  int m_tile, rest;
-  if (per_tile % 8 == 0) {
-    const int k = w >> 3;
-    m_tile = a.m_tiles - 1 - k % a.m_tiles;
-    rest = (w & 7) + 8 * (k / a.m_tiles);
-  } else {
-    m_tile = a.m_tiles - 1 - w / per_tile;
-    rest = w % per_tile;
-  }
-  const int b = rest / (a.Hkv * n_quads);
-  const int hkv = (rest / n_quads) % a.Hkv;
-  const int quad = rest % n_quads;
+  const int rows_per_block = 32 * (4 / GP);
+  const WorkItem item = a.live > 0 ? packed_item<CAUSAL>(w, a.cu, a.B, a.total, a.S, rows_per_block, a.Hkv * n_quads)
+                                   : dense_item<CAUSAL>(w, per_tile, a.Hkv * n_quads, a.m_tiles, a.S % rows_per_block != 0);
+  if (item.seq < 0) return;  // whole block, before any barrier
+  const int m_tile = item.tile, b = item.seq;
+  const int hkv = item.group / n_quads;
+  const int quad = item.group % n_quads;
   // key group (NG > 1) and wave within it
   const int kgrp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & (NG == 1 ? ~0 : 3);
   const int hq = hkv * G + quad * GP + wave_id % GP;
-  const int rows_per_block = 32 * (4 / GP);
 
   // this block's sequence: all of it for a dense batch; tokens [cu[b], cu[b+1])
   // of a packed one (clamped, so a malformed table cannot address past `total`)
@@ -459,6 +448,30 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
     landed();
     __syncthreads();
   };
+  if (NG == 1 && wave_first >= S) {
+    // A wave without rows only loads its share of the tiles, in both sweeps.
+    // (Ending a causal wave's steps at its own rows' last tile as well cost the
+    // others their registers: 168 -> 230 VGPRs at D 128.)
+    for (int t = 0; t < n_steps; ++t) {
+      dma_k(min(t + 2, n_tiles), t & 1);
+      dma_v(min(t + 1, n_tiles - 1), (t & 1) ^ 1);
+      landed();
+      __syncthreads();
+    }
+    if (__syncthreads_or(false)) {
+      dma_k(0, 0);
+      dma_v(0, 0);
+      landed();
+      __syncthreads();
+      for (int u = 0; u < n_tiles; ++u) {
+        dma_k(min(u + 1, n_tiles - 1), (u + 1) & 1);
+        dma_v(min(u + 1, n_tiles - 1), (u + 1) & 1);
+        landed();
+        __syncthreads();
+      }
+    }
+    return;
+  }
   for (int t = 0;;) {
     step(t, std::integral_constant<int, 0>{});
     if (++t >= n_steps) break;
@@ -556,9 +569,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
   }
 }
 
+// Blocks of the 16-bit kernels.
+int64_t fwd_blocks(const AttnArgs& a) { return (a.live > 0 ? a.live : (int64_t)a.m_tiles * a.B) * (a.Hq / a.gp); }
+
 template <typename T, int D, int KS, int NG>
 int launch_groups(const AttnArgs& a, bool causal, hipStream_t s) {
-  const int64_t blocks = (int64_t)a.m_tiles * a.B * a.Hq / a.gp;
+  const int64_t blocks = fwd_blocks(a);
   if (causal)
     hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, KS, NG>), dim3(blocks), dim3(NG * NT), 0, s, a);
   else
@@ -578,23 +594,16 @@ int launch_groups(const AttnArgs& a, bool causal, hipStream_t s) {
 //                      D 192, 128 tiles 130 -> 113; D 64, 64 tiles 35.3 -> 39.5
 //   two, full:         D 128, 64 tiles 66.9 -> 79.8 (the blocks are equally long and two share a CU)
 //   four:              D 128, 128 tiles causal 134 -> 155
-template <int D> bool split_keys(const AttnArgs& a, int64_t blocks, bool causal) {
+template <int D> bool split_keys(const AttnArgs& a, bool causal) {
   const int tiles = (a.S + BN - 1) / BN;
-  // packed sequences: at most one partial q tile each beside the whole ones
-  if (a.cu != nullptr) {
-    const int64_t rows = 32 * (4 / a.gp);
-    const int64_t live = (a.total / rows + a.B) * (a.Hq / a.gp);
-    blocks = live < blocks ? live : blocks;
-  }
-  const int64_t cus = cu_count();
+  const int64_t blocks = fwd_blocks(a), cus = cu_count();
   if (blocks <= cus) return tiles >= (D <= 64 ? 32 : 48);
   return blocks <= 2 * cus && causal && tiles >= (D <= 64 ? 192 : 96);
 }
 
 template <typename T, int D, int KS>
 int launch_ks(const AttnArgs& a, bool causal, hipStream_t s) {
-  const int64_t blocks = (int64_t)a.m_tiles * a.B * a.Hq / a.gp;
-  return split_keys<D>(a, blocks, causal) ? launch_groups<T, D, KS, kGroups<D>>(a, causal, s)
+  return split_keys<D>(a, causal) ? launch_groups<T, D, KS, kGroups<D>>(a, causal, s)
                                           : launch_groups<T, D, KS, 1>(a, causal, s);
 }
 
@@ -668,6 +677,7 @@ int attn_launch(const char* who, AttnArgs a, const int64_t* strides, int64_t bat
   const int64_t reach = (seq + 3 * BN) * (strides[4] > strides[7] ? strides[4] : strides[7]) * 2 + head_dim * 2;
   if (dtype != PK_F32 && reach > INT32_MAX)
     return fail(PK_ERR_UNSUPPORTED, "%s: K/V rows span more than 2 GiB per head", who);
+  a.live = dtype == PK_F32 ? 0 : packed_tiles(a.cu != nullptr, batch, a.total, seq, 32 * (4 / a.gp));
   a.c = fmaxf(fabsf(softmax_scale) * 1.4426950408889634f, 1e-30f);
   a.q_flip = softmax_scale < 0.f ? 0x80008000u : 0u;
   a.dr = (int)head_dim;
