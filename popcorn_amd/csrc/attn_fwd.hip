@@ -148,8 +148,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
   // their own, which the compiler can tell apart; with several they share one
   // area with the sums the groups hand over at the end.
   constexpr int KT = BN * KST, VT = BN * D;
-  constexpr int kMerge = 4 * (DT * 16 + 1) * 64;  // floats one group hands over: O^T and l of four waves
-  constexpr int kArea = NG == 1 ? 16 : max_of(NG * 2 * (KT + VT) * (int)sizeof(T), (NG - 1) * kMerge * 4);
+  constexpr int kMerge = 4 * DT * 16 * 64;  // floats of O^T that one group hands over (four waves), and NT of l
+  constexpr int kArea = NG == 1 ? 16 : max_of(NG * 2 * (KT + VT) * (int)sizeof(T), (NG - 1) * (kMerge + NT) * 4);
   __shared__ __attribute__((aligned(16))) T Ks1[NG == 1 ? 2 * KT : 8];
   __shared__ __attribute__((aligned(16))) T Vs1[NG == 1 ? 2 * VT : 8];
   __shared__ __attribute__((aligned(16))) unsigned char area[kArea];
@@ -481,25 +481,35 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
   if constexpr (NG > 1) {
     // groups 1 .. NG - 1 leave O^T and l in LDS (the tiles are done with: the
     // last step ended with a barrier); group 0 adds them in order
-    float* mine = reinterpret_cast<float*>(area) + wave * (DT * 16 + 1) * 64 + lane;
+    // (16 bytes a lane at a time: as single words the exchange took longer than
+    // two steps)
+    float4* mine = reinterpret_cast<float4*>(area) + wave * DT * 4 * 64 + lane;
+    float* lsum = reinterpret_cast<float*>(area) + (NG - 1) * kMerge + wave * 64 + lane;
     if (kgrp > 0) {
-      float* out = mine + (kgrp - 1) * kMerge;
+      float4* out = mine + (kgrp - 1) * (kMerge / 4);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) out[(dt * 16 + r) * 64] = acc[dt][r];
-      out[DT * 16 * 64] = l_i;
+        for (int r = 0; r < 4; ++r)
+          out[(dt * 4 + r) * 64] = make_float4(acc[dt][4 * r], acc[dt][4 * r + 1], acc[dt][4 * r + 2], acc[dt][4 * r + 3]);
+      lsum[(kgrp - 1) * NT] = l_i;
     }
     __syncthreads();
     if (kgrp == 0) {
 #pragma unroll
       for (int k = 0; k < NG - 1; ++k) {
-        const float* in = mine + k * kMerge;
+        const float4* in = mine + k * (kMerge / 4);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[dt][r] += in[(dt * 16 + r) * 64];
-        l_i += in[DT * 16 * 64];
+          for (int r = 0; r < 4; ++r) {
+            const float4 x = in[(dt * 4 + r) * 64];
+            acc[dt][4 * r] += x.x;
+            acc[dt][4 * r + 1] += x.y;
+            acc[dt][4 * r + 2] += x.z;
+            acc[dt][4 * r + 3] += x.w;
+          }
+        l_i += lsum[k * NT];
       }
     }
   }
@@ -584,21 +594,22 @@ int launch_groups(const AttnArgs& a, bool causal, hipStream_t s) {
 
 // Whether to split a block's keys over kGroups<D> key groups. The split block
 // has a CU to itself and walks its tiles kGroups times faster, but pays about
-// 5 us once (the wider block's start and the sum over the groups), and its
-// groups share every barrier. So it is for grids that cannot fill the CUs with
-// blocks of one group, and rows long enough to earn the cost back. Measured
+// 4.5 us once (D 128; the wider block's start and the sum over the groups), and
+// its groups share every barrier. So it is for grids that cannot fill the CUs
+// with blocks of one group, and rows long enough to earn the cost back. Measured
 // (us, one group -> split; bf16):
-//   one block per CU:  D 128, 256 tiles causal 169 -> 103; 32 tiles full 24.7 -> 25.3;
-//                      D 64, 64 tiles causal 31.0 -> 22.8, 33 tiles full 17.8 -> 15.9
-//   two, causal:       D 128, 512 tiles 377 -> 265, 64 tiles 53.4 -> 50.2;
-//                      D 192, 128 tiles 130 -> 113; D 64, 64 tiles 35.3 -> 39.5
-//   two, full:         D 128, 64 tiles 66.9 -> 79.8 (the blocks are equally long and two share a CU)
-//   four:              D 128, 128 tiles causal 134 -> 155
+//   one block per CU:  D 128 causal, 256 tiles 167 -> 102, 32 tiles 26.1 -> 24.3, 16 tiles 15.8 -> 17.1;
+//                      full, 32 tiles 25.0 -> 25.0; D 64, causal 64 tiles 31.0 -> 22.4, 16 tiles
+//                      11.2 -> 11.0, full 33 tiles 17.4 -> 15.5
+//   two, causal:       D 128, 512 tiles 372 -> 261, 64 tiles 53.2 -> 49.4; D 96, 64 tiles 42.1 -> 41.1;
+//                      D 192, 128 tiles 132 -> 113; D 256, 64 tiles 84.1 -> 83.0; D 64, 64 tiles 35.3 -> 38.4
+//   two, full:         D 128, 64 tiles 66.7 -> 79.2 (the blocks are equally long and two share a CU)
+//   four:              D 128, 128 tiles causal 133 -> 155
 template <int D> bool split_keys(const AttnArgs& a, bool causal) {
   const int tiles = (a.S + BN - 1) / BN;
   const int64_t blocks = fwd_blocks(a), cus = cu_count();
-  if (blocks <= cus) return tiles >= (D <= 64 ? 32 : 48);
-  return blocks <= 2 * cus && causal && tiles >= (D <= 64 ? 192 : 96);
+  if (blocks <= cus) return tiles >= (D <= 64 ? 24 : (causal ? 28 : 48));
+  return blocks <= 2 * cus && causal && tiles >= (D <= 64 ? 192 : 64);
 }
 
 template <typename T, int D, int KS>
