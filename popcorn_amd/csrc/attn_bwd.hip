@@ -32,9 +32,9 @@
 //               arrive through six LDS stages, two tiles in flight beyond the
 //               three a step reads. A block walks its q heads' tiles one
 //               after another, so when the grid is too small to fill the
-//               device the q heads of each group are split over several blocks
-//               that leave fp32 partials, and a third kernel adds them in
-//               split order (still deterministic).
+//               device the q heads of each group, and past them the query
+//               tiles, are split over several blocks that leave fp32 partials,
+//               and a third kernel adds them in order (still deterministic).
 //
 // Both kernels stage tiles with buffer loads that write LDS directly (16
 // bytes per lane at the wave's LDS base + 16 * lane): each lane fetches the
@@ -69,7 +69,10 @@ namespace {
 
 using namespace attn;
 
-constexpr int NT = 256;
+constexpr int NT = 256;  // threads of the dq kernel, or of each of its key groups
+constexpr int max_of(int a, int b) { return a > b ? a : b; }
+// Key groups of the split dq kernel: as many waves per SIMD as the rows' registers allow.
+template <int D> constexpr int kDqGroups = D <= 32 ? 4 : (D <= 64 ? 3 : (D <= 128 ? 2 : 1));
 constexpr int BM = 128;  // dq kernel: query rows per block times q heads per block
 constexpr int BN = 32;   // dq kernel: keys per tile
 constexpr int BK = 128;  // dkdv kernel: keys per block
@@ -93,6 +96,10 @@ struct BwdArgs {
   // packed), summed in split order by dkdv_sum_kernel
   float* part;
   int nsplit;
+  // The 16-bit dkdv kernel up to 128 dims also splits a block's query tiles into
+  // qsplit runs; parts = nsplit * qsplit blocks share a (key tile, kv head), and
+  // part is [parts][2]..., summed in that order.
+  int qsplit, parts;
   int64_t rows;
   int B, S, Hq, Hkv, group;
   int live_q, live_k;  // packed sequences: q and key tiles per group that the grids hold (packed_item), or 0
@@ -147,8 +154,11 @@ __device__ __forceinline__ uint4 flip(uint4 v, uint32_t f) { return make_uint4(v
 // KS: 16-dim steps of the S and dP products, D / 16, or one fewer when the
 // row's last 16 dims are all past head_dim (zeros in every operand of that
 // step, so skipping it changes no bit)
-template <typename T, int D, bool CAUSAL, int KS = D / 16>
-__global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_eu(D >= 192 ? 1 : 2))) void attn_bwd_dq_kernel(
+// NG: key groups, as in the forward: with more than one the block is NG times as
+// wide, each group of 4 waves holds the same rows and walks every NG-th key tile
+// through its own stages, and the groups' dQ are added through LDS at the end.
+template <typename T, int D, bool CAUSAL, int KS = D / 16, int NG = 1>
+__global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_waves_per_eu(D >= 192 ? 1 : 2))) void attn_bwd_dq_kernel(
     BwdArgs a) {
   using Frag = typename Mma<T>::frag;
   using L = Tile<D>;
@@ -163,8 +173,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   constexpr int DT = D / 32;
   constexpr int NSQ = 4;  // K/V tile stages: the two tiles a step reads, one in flight, one landing
   static_assert(KS == KK || KS == KK - 1, "at most the last 16-dim step is skipped");
-  __shared__ __attribute__((aligned(16))) T Ks[NSQ][BN * L::ST];
-  __shared__ __attribute__((aligned(16))) T Vs[NSQ][BN * L::ST];
+  // each key group's stages; with several groups they share one area with the
+  // dQ that the groups hand over at the end
+  constexpr int TILE = BN * L::ST;
+  constexpr int kMerge = 4 * DT * 16 * 64;  // floats of dQ^T that one group hands over (four waves)
+  constexpr int kArea = NG == 1 ? 16 : max_of(NG * 2 * NSQ * TILE * (int)sizeof(T), (NG - 1) * kMerge * 4);
+  __shared__ __attribute__((aligned(16))) T Ks1[NG == 1 ? NSQ * TILE : 8];
+  __shared__ __attribute__((aligned(16))) T Vs1[NG == 1 ? NSQ * TILE : 8];
+  __shared__ __attribute__((aligned(16))) unsigned char area[kArea];
   __shared__ __attribute__((aligned(16))) T spill[TFULL ? 8 : 64 * 8];
 
   // work item: (q tile, batch, kv head, head quad), longest causal rows
@@ -183,14 +199,24 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   if (item.seq < 0) return;  // whole block, before any barrier
   const int m_tile = item.tile, b = item.seq;
   const int hkv = item.group / n_quads;
-  const int hq = hkv * G + (item.group % n_quads) * GP + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % GP;
+  const int kgrp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // key group
+  const int hq = hkv * G + (item.group % n_quads) * GP +
+                 (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & (NG == 1 ? ~0 : 3)) % GP;
   int start, S;
   seq_bounds(a, b, start, S);
   const int m0 = m_tile * rows_per_block;
   if (m0 >= S) return;  // whole block, before any barrier
 
-  const int tid = threadIdx.x;
+  const int tid = NG == 1 ? threadIdx.x : threadIdx.x & (NT - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto kst = [&](int st) -> T* {
+    if constexpr (NG == 1) return Ks1 + st * TILE;
+    else return reinterpret_cast<T*>(area) + (kgrp * 2 * NSQ + st) * TILE;
+  };
+  auto vst = [&](int st) -> T* {
+    if constexpr (NG == 1) return Vs1 + st * TILE;
+    else return reinterpret_cast<T*>(area) + (kgrp * 2 * NSQ + NSQ + st) * TILE;
+  };
   const int lane = tid & 63;
   const int r32 = lane & 31;
   const int g = lane >> 5;
@@ -236,7 +262,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   const int64_t lidx = b * a.lse_bs + hq * a.lse_hs + start + q_row;
   // rows past the end: lse2 = +inf makes every p zero
   const float lse2 = row_ok ? a.lse[lidx] * 1.4426950408889634f : INFINITY;
-  if (row_ok && g == 0) {
+  if (row_ok && g == 0 && kgrp == 0) {
     a.dsum[lidx] = dsum;
     a.dsum[a.lse_n + lidx] = lse2;
   }
@@ -248,6 +274,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
 
   const int kv_end = CAUSAL ? min(m0 + rows_per_block, S) : S;
   const int n_tiles = (kv_end + BN - 1) / BN;
+  // key group k takes tiles k, k + NG, ...: all groups take the same number of
+  // steps, tiles past the end being the last one again with every key masked
+  const int n_own = NG == 1 ? n_tiles : (n_tiles + NG - 1) / NG;
+  auto tile_of = [&](int j) { return NG == 1 ? j : kgrp + NG * j; };
 
   // staging straight into LDS: slot i*NT + tid of a tile is row sl / KCH,
   // stored chunk sl % KCH, which holds logical chunk (sl % KCH) ^ swz(row)
@@ -263,8 +293,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
       const bool in = TFULL || i * NT + wave * 64 < TSLOTS;  // wave-uniform
-      T* kl = in ? Ks[buf] + (i * NT + wave * 64) * 8 : spill;
-      T* vl = in ? Vs[buf] + (i * NT + wave * 64) * 8 : spill;
+      T* kl = in ? kst(buf) + (i * NT + wave * 64) * 8 : spill;
+      T* vl = in ? vst(buf) + (i * NT + wave * 64) * 8 : spill;
       const int ko = t * BN * (int)a.ks[1] * (int)sizeof(T), vo = t * BN * (int)a.vs[1] * (int)sizeof(T);
       if constexpr (kAsmLoads) {
         ld_lds16_asm(kwords, kl, kgo[i], ko);
@@ -300,7 +330,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   // Tile indices are clamped into the range at the edges, where dS is zero.
   // (Tiles wholly past a wave's rows are masked to zero, not skipped.)
 #pragma unroll
-  for (int j = 0; j < NSQ - 2; ++j) issue(min(j, n_tiles - 1), j);
+  for (int j = 0; j < NSQ - 2; ++j) issue(min(tile_of(j), n_tiles - 1), j);
   lds_loads_landed();  // all of them: the dsum stores above share the counter
   __syncthreads();
   // product 3h: dQ step h (A = K^T from transposing reads of the tile at ka:
@@ -354,7 +384,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   auto dscores = [&](int u, Frag (&dsf)[2]) {
     // dS = P (dP - D), P = exp2(s c - lse2); keys a row must not see get 0.
     // The test for a mask is wave-uniform, so unmasked tiles branch past it.
-    const int kv0 = u * BN;
+    const int kv0 = tile_of(u) * BN;
     const bool need_mask = (CAUSAL && kv0 + BN - 1 > wave_first) || kv0 + BN > S;
     if (need_mask) {
 #pragma unroll
@@ -386,26 +416,26 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   };
   {
     // step 0: no dS yet (zero factors against the loaded stage 0); S^T, dP^T of tile 0
-    issue(min(NSQ - 2, n_tiles - 1), NSQ - 2);
+    issue(min(tile_of(NSQ - 2), n_tiles - 1), NSQ - 2);
     Frag dsf[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int j = 0; j < 8; ++j) dsf[c][j] = (T)0.f;
-    run(Ks[0], dsf, Ks[0], Vs[0]);
+    run(kst(0), dsf, kst(0), vst(0));
     finish();
   }
   auto step = [&](int t, auto phase) {
     constexpr int P = decltype(phase)::value;
     constexpr int PA = (P + NSQ - 1) % NSQ;
-    issue(min(t + NSQ - 2, n_tiles - 1), (P + NSQ - 2) % NSQ);
+    issue(min(tile_of(t + NSQ - 2), n_tiles - 1), (P + NSQ - 2) % NSQ);
     Frag dsf[2];
     dscores(t - 1, dsf);
-    run(Ks[PA], dsf, Ks[P], Vs[P]);  // dQ^T += K^T dS^T; S^T, dP^T of the next tile
+    run(kst(PA), dsf, kst(P), vst(P));  // dQ^T += K^T dS^T; S^T, dP^T of the next tile
     finish();
   };
   static_assert(NSQ == 4, "the step loop is unrolled over four stage phases");
-  if (wave_first >= S) {  // a wave without rows: only its share of the loads
+  if (NG == 1 && wave_first >= S) {  // a wave without rows: only its share of the loads
     for (int t = 1; t <= n_tiles; ++t) {
       issue(min(t + NSQ - 2, n_tiles - 1), (t + NSQ - 2) % NSQ);
       finish();
@@ -415,15 +445,41 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT, NT), amdgpu_waves_per_
   }
   for (int t = 1;;) {
     step(t, std::integral_constant<int, 1>{});
-    if (++t > n_tiles) break;
+    if (++t > n_own) break;
     step(t, std::integral_constant<int, 2>{});
-    if (++t > n_tiles) break;
+    if (++t > n_own) break;
     step(t, std::integral_constant<int, 3>{});
-    if (++t > n_tiles) break;
+    if (++t > n_own) break;
     step(t, std::integral_constant<int, 0>{});
-    if (++t > n_tiles) break;
+    if (++t > n_own) break;
   }
-  lds_loads_landed();  // tiles issued past the end, before the block's LDS is released
+  lds_loads_landed();  // tiles issued past the end, before the block's LDS is released or reused
+  if constexpr (NG > 1) {
+    __syncthreads();
+    float4* mine = reinterpret_cast<float4*>(area) + wave * DT * 4 * 64 + lane;
+    if (kgrp > 0) {
+      float4* out = mine + (kgrp - 1) * (kMerge / 4);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          out[(dt * 4 + r) * 64] = make_float4(acc[dt][4 * r], acc[dt][4 * r + 1], acc[dt][4 * r + 2], acc[dt][4 * r + 3]);
+    }
+    __syncthreads();
+    if (kgrp > 0) return;
+#pragma unroll
+    for (int k = 0; k < NG - 1; ++k)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float4 x = mine[k * (kMerge / 4) + (dt * 4 + r) * 64];
+          acc[dt][4 * r] += x.x;
+          acc[dt][4 * r + 1] += x.y;
+          acc[dt][4 * r + 2] += x.z;
+          acc[dt][4 * r + 3] += x.w;
+        }
+  }
 
   if (row_ok) {
     T* drow = static_cast<T*>(a.dq) + b * a.dqs[0] + hq * a.dqs[2] + (int64_t)(start + q_row) * a.dqs[1];
@@ -478,19 +534,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   // and the 32 resident blocks of one group start at 32 different places.)
   int kv_tile, b, group;
   if (a.live_k > 0) {
-    const WorkItem item = packed_item<false>(blockIdx.x, a.cu, a.B, a.total, a.S, BK, a.Hkv * a.nsplit);
+    const WorkItem item = packed_item<false>(blockIdx.x, a.cu, a.B, a.total, a.S, BK, a.Hkv * a.parts);
     if (item.seq < 0) return;  // whole block, before any barrier
     kv_tile = item.tile;
     b = item.seq;
     group = item.group;
   } else {
-    const int per_tile = a.B * a.Hkv * a.nsplit;
+    const int per_tile = a.B * a.Hkv * a.parts;
     kv_tile = blockIdx.x / per_tile;
-    b = blockIdx.x % per_tile / (a.Hkv * a.nsplit);
-    group = blockIdx.x % (a.Hkv * a.nsplit);
+    b = blockIdx.x % per_tile / (a.Hkv * a.parts);
+    group = blockIdx.x % (a.Hkv * a.parts);
   }
-  const int hkv = group / a.nsplit;
-  const int split = group % a.nsplit;
+  const int hkv = group / a.parts;
+  const int part = group % a.parts;
+  const int split = part / a.qsplit;  // of the q heads
   const int heads = a.group / a.nsplit;  // q heads this block walks, from split * heads on
   int start, S;
   seq_bounds(a, b, start, S);
@@ -529,8 +586,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   const float cs = a.q_flip ? -a.c : a.c;
 
   // query tiles: every q head of the group, rows from the block's first key on (causal)
-  const int u0 = CAUSAL ? kb0 / BQ : 0;
-  const int n_u = (S + BQ - 1) / BQ - u0;
+  // (with split query tiles, this block's run of them, which may be empty)
+  const int all_u0 = CAUSAL ? kb0 / BQ : 0;
+  const int all_u = (S + BQ - 1) / BQ - all_u0, piece = part % a.qsplit;
+  const int u0 = all_u0 + (int)((int64_t)all_u * piece / a.qsplit);
+  const int n_u = all_u0 + (int)((int64_t)all_u * (piece + 1) / a.qsplit) - u0;
   const int n_it = heads * n_u;
 
   // staging: slot sl = i*NT2 + tid of the stage (Q slots, then dO slots) is
@@ -782,10 +842,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
 
   if (key_ok) {
     const float f = role == 0 ? 1.0f : a.scale;  // dK: signed scale, Q was staged unflipped
-    if (a.nsplit > 1) {
-      // fp32 partial of this block's heads; dkdv_sum_kernel adds the splits
+    if (a.parts > 1) {
+      // fp32 partial of this block's heads and rows; dkdv_sum_kernel adds the parts
       const int64_t row = (a.cu != nullptr ? (int64_t)start : (int64_t)b * a.S) + key;
-      float* out = a.part + (((int64_t)(split * 2 + role) * a.rows + row) * a.Hkv + hkv) * D;
+      float* out = a.part + (((int64_t)(part * 2 + role) * a.rows + row) * a.Hkv + hkv) * D;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -809,7 +869,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
 }
 
 // dV (role 0) and dK (role 1) of one token row, kv head and 4 dims: the sum of
-// the nsplit partials in split order, rounded once. Rows are batch * S tokens
+// the partials in order, rounded once. Rows are batch * S tokens
 // (dense) or the packed token index.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void dkdv_sum_kernel(BwdArgs a) {
@@ -827,7 +887,7 @@ __global__ __launch_bounds__(256) void dkdv_sum_kernel(BwdArgs a) {
   for (int role = 0; role < 2; ++role) {
     const float* p = a.part + (int64_t)role * stride + (row * a.Hkv + hkv) * D + d4;
     float4 s = *reinterpret_cast<const float4*>(p);
-    for (int sp = 1; sp < a.nsplit; ++sp) {
+    for (int sp = 1; sp < a.parts; ++sp) {
       const float4 x = *reinterpret_cast<const float4*>(p + (int64_t)sp * 2 * stride);
       s.x += x.x;
       s.y += x.y;
@@ -853,19 +913,63 @@ int64_t dq_grid(BwdArgs& a) {
 #include "attn_bwd_f32.h"
 #include "attn_bwd_wide.h"
 
+// Whether the dq kernel splits its keys, by the rule of the forward (attn_fwd.hip,
+// split_keys). One pk_attn_bwd call, us, one group -> split (bf16, causal):
+//   one block per CU:  D 128, 256 tiles 444 -> 401, 64 tiles 118 -> 111, 32 tiles 90.0 -> 85.3 (one unit
+//                      of dq is not worth that: see split_keys), 16 tiles 55.2 -> 54.5;
+//                      D 64, 64 tiles 84.5 -> 78.4; full, 32 tiles 91.2 -> 91.2
+//   two:               D 128, 512 tiles 1005 -> 964, 128 tiles 295 -> 274, 64 tiles 173.1 -> 173.9;
+//                      D 64, 512 tiles 684 -> 611, 64 tiles 105 -> 111; full, 64 tiles 270 -> 284
+//   four:              D 128, 128 tiles 508 -> 530
+template <int D> bool split_dq(const BwdArgs& a, int64_t blocks, bool causal) {
+  const int tiles = (a.S + BN - 1) / BN;
+  const int64_t cus = cu_count();
+  if (blocks <= cus) return tiles >= (D <= 64 && causal ? 33 : 48);
+  return blocks <= 2 * cus && causal && tiles >= (D <= 64 ? 192 : 96);
+}
+
+// Number of q-head splits of the dk/dv kernel: the smallest divisor of the
+// group size that gives at least two blocks per CU, else the group size (one
+// q head per block). 1 keeps the direct path with no partials.
+int dkdv_splits(int64_t seqs, int64_t seq, int64_t kv_heads, int64_t group) {
+  const int64_t blocks = (seq + BK - 1) / BK * seqs * kv_heads;
+  const int64_t want = 2 * (int64_t)cu_count();
+  for (int64_t d = 1; d <= group; ++d)
+    if (group % d == 0 && (blocks * d >= want || d == group)) return (int)d;
+  return 1;
+}
+
+// Runs that a block's query tiles are split into where the q heads alone leave
+// CUs without a block, or (causal) with one: a causal grid of one block per CU
+// lasts as long as its first key tile's block, twice the average. Each run keeps
+// 32 tiles of the longest block, which its partials' traffic is worth.
+int dkdv_q_splits(int64_t seqs, int64_t seq, int64_t kv_heads, int64_t group, bool causal) {
+  const int64_t blocks = (seq + BK - 1) / BK * seqs * kv_heads * dkdv_splits(seqs, seq, kv_heads, group);
+  const int64_t want = (causal ? 2 : 1) * (int64_t)cu_count(), tiles = (seq + BQ - 1) / BQ;
+  int q = 1;
+  while (q < 8 && blocks * q < want && tiles >= 2 * q * 32) q *= 2;
+  return q;
+}
+
 template <typename T, int D, int KS>
 int launch_ks(BwdArgs a, bool causal, hipStream_t s) {
   const int64_t dq_blocks = dq_grid(a);
+  a.qsplit = dkdv_q_splits(a.B, a.S, a.Hkv, a.group, causal);
+  a.parts = a.nsplit * a.qsplit;
   a.live_k = packed_tiles(a.cu != nullptr, a.B, a.total, a.S, BK);
-  const int64_t kv_blocks = (a.live_k > 0 ? a.live_k : (int64_t)((a.S + BK - 1) / BK) * a.B) * a.Hkv * a.nsplit;
+  const int64_t kv_blocks = (a.live_k > 0 ? a.live_k : (int64_t)((a.S + BK - 1) / BK) * a.B) * a.Hkv * a.parts;
+  constexpr int NG = kDqGroups<D>;
+  const bool split = split_dq<D>(a, dq_blocks, causal);
   if (causal) {
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, KS>), dim3(dq_blocks), dim3(NT), 0, s, a);
+    if (split) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, KS, NG>), dim3(dq_blocks), dim3(NG * NT), 0, s, a);
+    else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, KS>), dim3(dq_blocks), dim3(NT), 0, s, a);
     hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, true, KS>), dim3(kv_blocks), dim3(NT2), 0, s, a);
   } else {
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, KS>), dim3(dq_blocks), dim3(NT), 0, s, a);
+    if (split) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, KS, NG>), dim3(dq_blocks), dim3(NG * NT), 0, s, a);
+    else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, KS>), dim3(dq_blocks), dim3(NT), 0, s, a);
     hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, false, KS>), dim3(kv_blocks), dim3(NT2), 0, s, a);
   }
-  if (a.nsplit > 1) {
+  if (a.parts > 1) {
     const int64_t n = a.rows * a.Hkv * (a.dr / 4);
     hipLaunchKernelGGL((dkdv_sum_kernel<T, D>), dim3((n + 255) / 256), dim3(256), 0, s, a);
   }
@@ -883,28 +987,24 @@ int launch(const BwdArgs& a, bool causal, hipStream_t s) {
   return launch_ks<T, D, D / 16>(a, causal, s);
 }
 
-// Number of q-head splits of the dk/dv kernel: the smallest divisor of the
-// group size that gives at least two blocks per CU, else the group size (one
-// q head per block). 1 keeps the direct path with no partials.
-int dkdv_splits(int64_t seqs, int64_t seq, int64_t kv_heads, int64_t group) {
-  const int64_t blocks = (seq + BK - 1) / BK * seqs * kv_heads;
-  const int64_t want = 2 * (int64_t)cu_count();
-  for (int64_t d = 1; d <= group; ++d)
-    if (group % d == 0 && (blocks * d >= want || d == group)) return (int)d;
-  return 1;
-}
-
 constexpr int64_t kAlign = 256;
 inline int64_t round_up(int64_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
+
+// Partials that a call needs room for: with the causal splits, which the others
+// do not exceed. (The query is not told of the mask or of fp32, which splits the
+// q heads only.)
+int dkdv_parts(int64_t seqs, int64_t seq, int64_t kv_heads, int64_t group, int64_t head_dim) {
+  return dkdv_splits(seqs, seq, kv_heads, group) * (head_dim <= 128 ? dkdv_q_splits(seqs, seq, kv_heads, group, true) : 1);
+}
 
 // Workspace bytes: D and lse2 (2 * lse_n floats), then the dk/dv partials when
 // the kernel splits the q heads.
 // (The partials are laid out at the kernels' row width: 64, 96, 128 or 256 dims; fp32, whose
 // kernels have no 96-dim layout, is counted at 128, which covers either.)
-int64_t workspace_bytes(int64_t lse_n, int64_t rows, int64_t kv_heads, int64_t head_dim, int nsplit) {
+int64_t workspace_bytes(int64_t lse_n, int64_t rows, int64_t kv_heads, int64_t head_dim, int parts) {
   const int64_t width = head_dim <= 64 ? 64 : (head_dim <= 128 ? 128 : 256);
-  const int64_t parts = nsplit > 1 ? (int64_t)nsplit * 2 * rows * kv_heads * width * (int64_t)sizeof(float) : 0;
-  return round_up(2 * lse_n * (int64_t)sizeof(float)) + parts;
+  const int64_t bytes = parts > 1 ? (int64_t)parts * 2 * rows * kv_heads * width * (int64_t)sizeof(float) : 0;
+  return round_up(2 * lse_n * (int64_t)sizeof(float)) + bytes;
 }
 
 // strides[24] = q, k, v, o, dout, dq, dk, dv (batch, token, head)
@@ -919,8 +1019,10 @@ int bwd_launch(const char* who, BwdArgs a, void* workspace, int64_t workspace_by
   if (kv_heads == 0 || q_heads % kv_heads != 0)
     return fail(PK_ERR_INVALID, "%s: q_heads=%lld is not a multiple of kv_heads=%lld", who, (long long)q_heads,
                 (long long)kv_heads);
-  a.nsplit = dkdv_splits(batch, seq, kv_heads, q_heads / kv_heads);
-  const int64_t need = workspace_bytes(a.lse_n, a.rows, kv_heads, head_dim, a.nsplit);
+  a.nsplit = a.parts = dkdv_splits(batch, seq, kv_heads, q_heads / kv_heads);
+  a.qsplit = 1;
+  const int64_t need = workspace_bytes(a.lse_n, a.rows, kv_heads, head_dim,
+                                       dkdv_parts(batch, seq, kv_heads, q_heads / kv_heads, head_dim));
   if (workspace_bytes_given < need)
     return fail(PK_ERR_INVALID, "%s: workspace of %lld bytes, %lld needed", who, (long long)workspace_bytes_given,
                 (long long)need);
@@ -992,8 +1094,8 @@ extern "C" {
 int64_t pk_attn_bwd_workspace(int64_t batch, int64_t seq, int64_t q_heads, int64_t kv_heads, int64_t head_dim) {
   using namespace pk;
   if (batch < 0 || seq < 0 || q_heads < 0 || kv_heads <= 0 || head_dim < 0 || q_heads % kv_heads != 0) return -1;
-  const int nsplit = dkdv_splits(batch, seq, kv_heads, q_heads / kv_heads);
-  return workspace_bytes(batch * q_heads * seq, batch * seq, kv_heads, head_dim, nsplit);
+  const int parts = dkdv_parts(batch, seq, kv_heads, q_heads / kv_heads, head_dim);
+  return workspace_bytes(batch * q_heads * seq, batch * seq, kv_heads, head_dim, parts);
 }
 
 int64_t pk_attn_varlen_bwd_workspace(int64_t num_seqs, int64_t total, int64_t max_seqlen, int64_t q_heads,
@@ -1002,8 +1104,8 @@ int64_t pk_attn_varlen_bwd_workspace(int64_t num_seqs, int64_t total, int64_t ma
   if (num_seqs < 0 || total < 0 || max_seqlen < 0 || q_heads < 0 || kv_heads <= 0 || head_dim < 0 ||
       q_heads % kv_heads != 0)
     return -1;
-  const int nsplit = dkdv_splits(num_seqs, max_seqlen, kv_heads, q_heads / kv_heads);
-  return workspace_bytes(q_heads * total, total, kv_heads, head_dim, nsplit);
+  const int parts = dkdv_parts(num_seqs, max_seqlen, kv_heads, q_heads / kv_heads, head_dim);
+  return workspace_bytes(q_heads * total, total, kv_heads, head_dim, parts);
 }
 
 int pk_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, const float* lse,

@@ -605,10 +605,14 @@ int launch_groups(const AttnArgs& a, bool causal, hipStream_t s) {
 //                      D 192, 128 tiles 132 -> 113; D 256, 64 tiles 84.1 -> 83.0; D 64, 64 tiles 35.3 -> 38.4
 //   two, full:         D 128, 64 tiles 66.7 -> 79.2 (the blocks are equally long and two share a CU)
 //   four:              D 128, 128 tiles causal 133 -> 155
+// A call that keeps its log-sum-exp for a backward splits only from rows on
+// where that backward's dq kernel does: below, a sequence then has the same
+// gradients, to a unit of its type, alone and in a batch that fills the grid.
 template <int D> bool split_keys(const AttnArgs& a, bool causal) {
   const int tiles = (a.S + BN - 1) / BN;
   const int64_t blocks = fwd_blocks(a), cus = cu_count();
-  if (blocks <= cus) return tiles >= (D <= 64 ? 24 : (causal ? 28 : 48));
+  const bool alone = a.lse == nullptr;
+  if (blocks <= cus) return tiles >= (D <= 64 ? (alone ? 24 : 32) : (alone && causal ? 28 : 48));
   return blocks <= 2 * cus && causal && tiles >= (D <= 64 ? 192 : 64);
 }
 
