@@ -102,6 +102,7 @@ struct BwdArgs {
   int qsplit, parts;
   int64_t rows;
   int B, S, Hq, Hkv, group;
+  int snake_q, snake_k;  // dense_item
   int live_q, live_k;  // packed sequences: q and key tiles per group that the grids hold (packed_item), or 0
   float scale;  // signed softmax scale
   float c;      // |scale| * log2(e), at least 1e-30
@@ -144,6 +145,23 @@ __device__ __forceinline__ void seq_bounds(const BwdArgs& a, int b, int& start, 
     start = min(max(a.cu[b], 0), a.total);
     S = min(min(max(a.cu[b + 1], start), a.total) - start, a.S);
   }
+}
+
+// Work item of a dk/dv kernel: (key tile, sequence, kv head and part), first key
+// tiles (the most causal work) first. (Group-major order per XCD, as the forward
+// and dq kernels use for dense batches, measured 26 % more HBM fetch here: a
+// block streams its group's whole Q/dO from its own key tile on, and the 32
+// resident blocks of one group start at 32 different places.)
+__device__ __forceinline__ WorkItem key_item(const BwdArgs& a, int w) {
+  const int per_seq = a.Hkv * a.parts;
+  if (a.live_k > 0) return packed_item<false>(w, a.cu, a.B, a.total, a.S, BK, per_seq);
+  if (a.snake_k > 0) {
+    const int tiles = (a.S + BK - 1) / BK;
+    const WorkItem item = dense_item<true>(w, a.B * per_seq, per_seq, tiles, false, a.snake_k);
+    return {item.seq, item.group, tiles - 1 - item.tile};
+  }
+  const int rest = w % (a.B * per_seq);
+  return {rest / per_seq, rest % per_seq, w / (a.B * per_seq)};
 }
 
 __device__ __forceinline__ uint4 flip(uint4 v, uint32_t f) { return make_uint4(v.x ^ f, v.y ^ f, v.z ^ f, v.w ^ f); }
@@ -195,7 +213,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
   const int w = blockIdx.x;
   const WorkItem item =
       a.live_q > 0 ? packed_item<CAUSAL>(w, a.cu, a.B, a.total, a.S, rows_per_block, a.Hkv * n_quads)
-                   : dense_item<CAUSAL>(w, a.B * a.Hkv * n_quads, a.Hkv * n_quads, m_tiles, a.S % rows_per_block != 0);
+                   : dense_item<CAUSAL>(w, a.B * a.Hkv * n_quads, a.Hkv * n_quads, m_tiles,
+                                            a.S % rows_per_block != 0, a.snake_q);
   if (item.seq < 0) return;  // whole block, before any barrier
   const int m_tile = item.tile, b = item.seq;
   const int hkv = item.group / n_quads;
@@ -528,25 +547,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   __shared__ __attribute__((aligned(16))) _Float16 Pb[2][4][16 * 64];
 
-  // first key tiles (the most causal work) first. (Group-major order per XCD,
-  // as the forward and dq kernels use for dense batches, measured 26 % more HBM
-  // fetch here: a block streams its group's whole Q/dO from its own key tile on,
-  // and the 32 resident blocks of one group start at 32 different places.)
-  int kv_tile, b, group;
-  if (a.live_k > 0) {
-    const WorkItem item = packed_item<false>(blockIdx.x, a.cu, a.B, a.total, a.S, BK, a.Hkv * a.parts);
-    if (item.seq < 0) return;  // whole block, before any barrier
-    kv_tile = item.tile;
-    b = item.seq;
-    group = item.group;
-  } else {
-    const int per_tile = a.B * a.Hkv * a.parts;
-    kv_tile = blockIdx.x / per_tile;
-    b = blockIdx.x % per_tile / (a.Hkv * a.parts);
-    group = blockIdx.x % (a.Hkv * a.parts);
-  }
-  const int hkv = group / a.parts;
-  const int part = group % a.parts;
+  const WorkItem item = key_item(a, blockIdx.x);
+  if (item.seq < 0) return;  // whole block, before any barrier
+  const int kv_tile = item.tile, b = item.seq;
+  const int hkv = item.group / a.parts;
+  const int part = item.group % a.parts;
   const int split = part / a.qsplit;  // of the q heads
   const int heads = a.group / a.nsplit;  // q heads this block walks, from split * heads on
   int start, S;
@@ -903,11 +908,25 @@ __global__ __launch_bounds__(256) void dkdv_sum_kernel(BwdArgs a) {
   }
 }
 
-// The 16-bit dq kernel's grid; sets which of its work mappings applies.
-int64_t dq_grid(BwdArgs& a) {
+// dense_item's snake: for causal grids of more than one block per CU, all resident at once.
+int snake_cus(bool causal, int64_t blocks, int resident) {
+  const int64_t cus = cu_count();
+  return causal && blocks > cus && blocks <= resident * cus ? (int)(cus / 8) : 0;
+}
+
+// The dq kernels' grid, of which `resident` blocks fit on a CU; sets which of their work mappings applies.
+int64_t dq_grid(BwdArgs& a, bool causal, int resident) {
   const int gp = a.group % 4 == 0 ? 4 : (a.group % 2 == 0 ? 2 : 1), rows = 32 * (4 / gp);
   a.live_q = packed_tiles(a.cu != nullptr, a.B, a.total, a.S, rows);
-  return (a.live_q > 0 ? a.live_q : (int64_t)((a.S + rows - 1) / rows) * a.B) * (a.Hq / gp);
+  const int64_t blocks = (a.live_q > 0 ? a.live_q : (int64_t)((a.S + rows - 1) / rows) * a.B) * (a.Hq / gp);
+  a.snake_q = snake_cus(causal, blocks, resident);
+  return blocks;
+}
+
+// A dk/dv kernel's grid (set a.parts first); sets which of its work mappings applies.
+int64_t key_grid(BwdArgs& a) {
+  a.live_k = packed_tiles(a.cu != nullptr, a.B, a.total, a.S, BK);
+  return (a.live_k > 0 ? a.live_k : (int64_t)((a.S + BK - 1) / BK) * a.B) * a.Hkv * a.parts;
 }
 
 #include "attn_bwd_f32.h"
@@ -953,13 +972,14 @@ int dkdv_q_splits(int64_t seqs, int64_t seq, int64_t kv_heads, int64_t group, bo
 
 template <typename T, int D, int KS>
 int launch_ks(BwdArgs a, bool causal, hipStream_t s) {
-  const int64_t dq_blocks = dq_grid(a);
+  const int64_t dq_blocks = dq_grid(a, causal, D <= 32 ? 4 : (D <= 64 ? 3 : 2));
   a.qsplit = dkdv_q_splits(a.B, a.S, a.Hkv, a.group, causal);
   a.parts = a.nsplit * a.qsplit;
-  a.live_k = packed_tiles(a.cu != nullptr, a.B, a.total, a.S, BK);
-  const int64_t kv_blocks = (a.live_k > 0 ? a.live_k : (int64_t)((a.S + BK - 1) / BK) * a.B) * a.Hkv * a.parts;
+  const int64_t kv_blocks = key_grid(a);
   constexpr int NG = kDqGroups<D>;
   const bool split = split_dq<D>(a, dq_blocks, causal);
+  if (split) a.snake_q = 0;
+  a.snake_k = snake_cus(causal, kv_blocks, D <= 64 ? 2 : 1);
   if (causal) {
     if (split) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, KS, NG>), dim3(dq_blocks), dim3(NG * NT), 0, s, a);
     else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, KS>), dim3(dq_blocks), dim3(NT), 0, s, a);

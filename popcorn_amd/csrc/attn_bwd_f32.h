@@ -132,21 +132,16 @@ void attn_bwd_f32_dq_kernel(BwdArgs a) {
   const int rows_per_block = 32 * (4 / GP);
   const int m_tiles = (a.S + rows_per_block - 1) / rows_per_block;
   const int n_quads = G / GP;
-  const int per_tile = a.B * a.Hkv * n_quads;
   const int w = blockIdx.x;
-  int m_tile, rest;
-  if (per_tile % 8 == 0) {  // group-major per XCD
-    const int k = w >> 3;
-    m_tile = m_tiles - 1 - k % m_tiles;
-    rest = (w & 7) + 8 * (k / m_tiles);
-  } else {
-    m_tile = m_tiles - 1 - w / per_tile;
-    rest = w % per_tile;
-  }
-  const int b = rest / (a.Hkv * n_quads);
-  const int hkv = (rest / n_quads) % a.Hkv;
+  const WorkItem item =
+      a.live_q > 0 ? packed_item<CAUSAL>(w, a.cu, a.B, a.total, a.S, rows_per_block, a.Hkv * n_quads)
+                   : dense_item<CAUSAL>(w, a.B * a.Hkv * n_quads, a.Hkv * n_quads, m_tiles, a.S % rows_per_block != 0,
+                                        a.snake_q);
+  if (item.seq < 0) return;  // whole block, before any barrier
+  const int m_tile = item.tile, b = item.seq;
+  const int hkv = item.group / n_quads;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int hq = hkv * G + (rest % n_quads) * GP + wave % GP;
+  const int hq = hkv * G + (item.group % n_quads) * GP + wave % GP;
   int start, S;
   seq_bounds(a, b, start, S);
   const int m0 = m_tile * rows_per_block;
@@ -316,12 +311,11 @@ void attn_bwd_f32_dkdv_kernel(BwdArgs a) {
   __shared__ __attribute__((aligned(16))) float4 Pb[2][4][4 * 64];  // P per slice: [buffer][slice][r / 4][lane]
 
   const int w = blockIdx.x;
-  const int per_tile = a.B * a.Hkv * a.nsplit;
-  const int kv_tile = w / per_tile;  // first key tiles (the most causal work) first
-  const int gi = w % per_tile;
-  const int b = gi / (a.Hkv * a.nsplit);
-  const int hkv = (gi / a.nsplit) % a.Hkv;
-  const int split = gi % a.nsplit;
+  const WorkItem item = key_item(a, w);
+  if (item.seq < 0) return;  // whole block, before any barrier
+  const int kv_tile = item.tile, b = item.seq;
+  const int hkv = item.group / a.nsplit;
+  const int split = item.group % a.nsplit;
   const int heads = a.group / a.nsplit;  // q heads this block walks, from split * heads on
   int start, S;
   seq_bounds(a, b, start, S);
@@ -512,12 +506,11 @@ void attn_bwd_f32_dkdv_wide_kernel(BwdArgs a) {
 
   const int half = blockIdx.x & 1;  // output dims 128 half .. 128 half + 127
   const int w = blockIdx.x >> 1;
-  const int per_tile = a.B * a.Hkv * a.nsplit;
-  const int kv_tile = w / per_tile;  // first key tiles (the most causal work) first
-  const int gi = w % per_tile;
-  const int b = gi / (a.Hkv * a.nsplit);
-  const int hkv = (gi / a.nsplit) % a.Hkv;
-  const int split = gi % a.nsplit;
+  const WorkItem item = key_item(a, w);
+  if (item.seq < 0) return;  // whole block, before any barrier
+  const int kv_tile = item.tile, b = item.seq;
+  const int hkv = item.group / a.nsplit;
+  const int split = item.group % a.nsplit;
   const int heads = a.group / a.nsplit;
   int start, S;
   seq_bounds(a, b, start, S);
@@ -672,10 +665,9 @@ void attn_bwd_f32_dkdv_wide_kernel(BwdArgs a) {
   }
 }
 
-template <int D> int launch_f32(const BwdArgs& a, bool causal, hipStream_t s) {
-  const int gp = a.group % 4 == 0 ? 4 : (a.group % 2 == 0 ? 2 : 1);
-  const int64_t dq_blocks = (int64_t)((a.S + 32 * (4 / gp) - 1) / (32 * (4 / gp))) * a.B * a.Hq / gp;
-  const int64_t kv_blocks = (int64_t)((a.S + BK - 1) / BK) * a.B * a.Hkv * a.nsplit;
+template <int D> int launch_f32(BwdArgs a, bool causal, hipStream_t s) {
+  const int64_t dq_blocks = dq_grid(a, causal, D <= 64 ? 2 : 1);
+  const int64_t kv_blocks = key_grid(a);
   if (causal)
     hipLaunchKernelGGL((attn_bwd_f32_dq_kernel<D, true>), dim3(dq_blocks), dim3(kF32DqThreads), 0, s, a);
   else

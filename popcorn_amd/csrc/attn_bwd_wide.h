@@ -35,12 +35,11 @@ void attn_bwd_dkdv_wide_kernel(BwdArgs a) {
   __shared__ __attribute__((aligned(16))) float RV[2][2][64];  // buffer: lse2 rows, D rows (32 used)
 
   const int w = blockIdx.x;
-  const int per_tile = a.B * a.Hkv * a.nsplit;
-  const int kv_tile = w / per_tile;  // first key tiles (the most causal work) first
-  const int gi = w % per_tile;
-  const int b = gi / (a.Hkv * a.nsplit);
-  const int hkv = (gi / a.nsplit) % a.Hkv;
-  const int split = gi % a.nsplit;
+  const WorkItem item = key_item(a, w);
+  if (item.seq < 0) return;  // whole block, before any barrier
+  const int kv_tile = item.tile, b = item.seq;
+  const int hkv = item.group / a.nsplit;
+  const int split = item.group % a.nsplit;
   const int heads = a.group / a.nsplit;  // q heads this block walks, from split * heads on
   int start, S;
   seq_bounds(a, b, start, S);
@@ -264,8 +263,8 @@ void attn_bwd_dkdv_wide_kernel(BwdArgs a) {
 
 // head_dim 136-256 in bf16 or fp16 (rows of D = 192 or 256): the dq kernel at D and the single-role dk/dv kernel
 template <typename T, int D> int launch_wide(BwdArgs a, bool causal, hipStream_t s) {
-  const int64_t dq_blocks = dq_grid(a);
-  const int64_t kv_blocks = (int64_t)((a.S + BK - 1) / BK) * a.B * a.Hkv * a.nsplit;
+  const int64_t dq_blocks = dq_grid(a, causal, 1);
+  const int64_t kv_blocks = key_grid(a);
   if (causal) {
     hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true>), dim3(dq_blocks), dim3(NT), 0, s, a);
     hipLaunchKernelGGL((attn_bwd_dkdv_wide_kernel<T, D, true>), dim3(kv_blocks), dim3(kWideThreads), 0, s, a);

@@ -118,6 +118,7 @@ struct AttnArgs {
   int64_t lse_bs, lse_hs;  // lse element (b, h, token t of b) at b*lse_bs + h*lse_hs + t (+ cu[b] when packed)
   int B, S, Hq, Hkv, group, m_tiles;
   int live;  // packed sequences: q tiles per group of heads that the grid holds (packed_item), or 0
+  int snake;  // dense_item
   int gp;  // q heads of one kv group per block (4, 2 or 1); the block's 4 waves are gp heads x 4/gp row groups
   float c;          // |scale| * log2(e), at least 1e-30
   uint32_t q_flip;  // 0x80008000 when scale < 0 (negates both halves of a packed pair), else 0
@@ -125,6 +126,15 @@ struct AttnArgs {
   // 16-byte chunks: the kernel lays rows out at D and reads zeros past them
   int dr, dch;
 };
+
+// Blocks of a call.
+int64_t fwd_blocks(const AttnArgs& a) { return (a.live > 0 ? a.live : (int64_t)a.m_tiles * a.B) * (a.Hq / a.gp); }
+
+// dense_item's snake: for causal grids of more than one block per CU, all resident at once.
+int snake_cus(bool causal, int64_t blocks, int resident) {
+  const int64_t cus = cu_count();
+  return causal && blocks > cus && blocks <= resident * cus ? (int)(cus / 8) : 0;
+}
 
 // NG: key groups. One is the kernel described above. With more, the block is NG
 // times as wide, each group of 4 waves holds the same rows and heads and walks
@@ -163,7 +173,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
   const int w = blockIdx.x;
   const int rows_per_block = 32 * (4 / GP);
   const WorkItem item = a.live > 0 ? packed_item<CAUSAL>(w, a.cu, a.B, a.total, a.S, rows_per_block, a.Hkv * n_quads)
-                                   : dense_item<CAUSAL>(w, per_tile, a.Hkv * n_quads, a.m_tiles, a.S % rows_per_block != 0);
+                                   : dense_item<CAUSAL>(w, per_tile, a.Hkv * n_quads, a.m_tiles, a.S % rows_per_block != 0, a.snake);
   if (item.seq < 0) return;  // whole block, before any barrier
   const int m_tile = item.tile, b = item.seq;
   const int hkv = item.group / n_quads;
@@ -579,12 +589,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
   }
 }
 
-// Blocks of the 16-bit kernels.
-int64_t fwd_blocks(const AttnArgs& a) { return (a.live > 0 ? a.live : (int64_t)a.m_tiles * a.B) * (a.Hq / a.gp); }
-
 template <typename T, int D, int KS, int NG>
-int launch_groups(const AttnArgs& a, bool causal, hipStream_t s) {
+int launch_groups(AttnArgs a, bool causal, hipStream_t s) {
   const int64_t blocks = fwd_blocks(a);
+  a.snake = snake_cus(causal, blocks, NG > 1 ? 1 : (D <= 64 ? 4 : (D <= 128 ? 3 : 2)));
   if (causal)
     hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, KS, NG>), dim3(blocks), dim3(NG * NT), 0, s, a);
   else
@@ -692,7 +700,7 @@ int attn_launch(const char* who, AttnArgs a, const int64_t* strides, int64_t bat
   const int64_t reach = (seq + 3 * BN) * (strides[4] > strides[7] ? strides[4] : strides[7]) * 2 + head_dim * 2;
   if (dtype != PK_F32 && reach > INT32_MAX)
     return fail(PK_ERR_UNSUPPORTED, "%s: K/V rows span more than 2 GiB per head", who);
-  a.live = dtype == PK_F32 ? 0 : packed_tiles(a.cu != nullptr, batch, a.total, seq, 32 * (4 / a.gp));
+  a.live = packed_tiles(a.cu != nullptr, batch, a.total, seq, 32 * (4 / a.gp));
   a.c = fmaxf(fabsf(softmax_scale) * 1.4426950408889634f, 1e-30f);
   a.q_flip = softmax_scale < 0.f ? 0x80008000u : 0u;
   a.dr = (int)head_dim;

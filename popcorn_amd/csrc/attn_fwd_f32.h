@@ -45,21 +45,16 @@ void attn_fwd_f32_kernel(AttnArgs a) {
   const int n_quads = G / GP;
   const int per_tile = a.B * a.Hkv * n_quads;
   const int w = blockIdx.x;
-  int m_tile, rest;
-  if (per_tile % 8 == 0) {
-    const int k = w >> 3;
-    m_tile = a.m_tiles - 1 - k % a.m_tiles;
-    rest = (w & 7) + 8 * (k / a.m_tiles);
-  } else {
-    m_tile = a.m_tiles - 1 - w / per_tile;
-    rest = w % per_tile;
-  }
-  const int b = rest / (a.Hkv * n_quads);
-  const int hkv = (rest / n_quads) % a.Hkv;
-  const int quad = rest % n_quads;
+  const int rows_per_block = 32 * (4 / GP);
+  const WorkItem item = a.live > 0 ? packed_item<CAUSAL>(w, a.cu, a.B, a.total, a.S, rows_per_block, a.Hkv * n_quads)
+                                   : dense_item<CAUSAL>(w, per_tile, a.Hkv * n_quads, a.m_tiles,
+                                                        a.S % rows_per_block != 0, a.snake);
+  if (item.seq < 0) return;  // whole block, before any barrier
+  const int m_tile = item.tile, b = item.seq;
+  const int hkv = item.group / n_quads;
+  const int quad = item.group % n_quads;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hq = hkv * G + quad * GP + wave % GP;
-  const int rows_per_block = 32 * (4 / GP);
 
   int S = a.S, start = 0;
   if (a.cu != nullptr) {
@@ -228,8 +223,9 @@ void attn_fwd_f32_kernel(AttnArgs a) {
   }
 }
 
-template <int D> int launch_f32(const AttnArgs& a, int causal, hipStream_t s) {
-  const int blocks = a.m_tiles * a.B * a.Hq / a.gp;
+template <int D> int launch_f32(AttnArgs a, int causal, hipStream_t s) {
+  const int64_t blocks = fwd_blocks(a);
+  a.snake = snake_cus(causal, blocks, D == 256 ? 1 : 2);
   if (causal)
     hipLaunchKernelGGL((attn_fwd_f32_kernel<D, true>), dim3(blocks), dim3(kF32Threads), 0, s, a);
   else
