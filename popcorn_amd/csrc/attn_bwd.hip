@@ -532,7 +532,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   // issues the same loads and its vmcnt counts hold
   constexpr bool TFULL = 2 * SLOTS % NT2 == 0;
   constexpr int NS = 6;                  // query tiles resident or in flight in LDS
-  constexpr int PER_ISSUE = TI + 1;      // loads each wave issues per tile (tiles, one row vector)
   constexpr int TILE = BQ * D;
   constexpr int KK = D / 16;
   constexpr int DT = D / 32;
@@ -540,7 +539,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   // stage: Q tile then dO tile; row vectors: lse2, then D (64 slots: whole-wave loads)
   __shared__ __attribute__((aligned(16))) T QG[NS][2 * TILE];
   __shared__ __attribute__((aligned(16))) float RV[NS][2][64];
-  __shared__ __attribute__((aligned(16))) float spill[64];
   __shared__ __attribute__((aligned(16))) T tspill[TFULL ? 8 : 64 * 8];
   // P of each key slice as fp16 (P <= 1; 11 significant bits, more than the
   // rounded dS it feeds), double-buffered: [buffer][slice][16 values x 64 lanes]
@@ -613,7 +611,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   // the group) and q tile, and the buffer descriptors of that head, rebuilt
   // only when the head changes; past the end the last tile is issued again.
   // Rows past the end read as zero; their p is masked. Wave 0 also loads the
-  // rows' lse2, wave 1 their D, the other waves repeat D into `spill`.
+  // rows' lse2 and wave 1 their D; the waits allow the TI loads an issue that
+  // every wave has, so those two wait for up to two loads more. Against the
+  // other waves loading D once more to no use: 7747 -> 7678 us at B4 T8192
+  // H32/8 D128 causal, 956 -> 949 at B2 T4096, no change at D64.
   int cur_h = 0, cur_u = 0, cur_it = 0;
   __amdgpu_buffer_rsrc_t trs[TI], rrs;
   int tstride[TI];  // bytes per row of the tensor each of this wave's tile loads reads
@@ -642,8 +643,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
       const bool in = TFULL || i * NT2 + wave * 64 < 2 * SLOTS;  // wave-uniform
       ld_buf_lds(trs[i], in ? QG[st] + (i * NT2 + wave * 64) * 8 : tspill, go[i], r0 * tstride[i]);
     }
-    ld_buf_lds4(rrs, wave == 0 ? RV[st][0] : (wave == 1 ? RV[st][1] : spill), lane * (int)sizeof(float),
-                r0 * (int)sizeof(float));
+    if (wave < 2)
+      ld_buf_lds4(rrs, RV[st][wave], lane * (int)sizeof(float), r0 * (int)sizeof(float));
     if (cur_it + 1 < n_it) {
       ++cur_it;
       if (++cur_u == n_u) {
@@ -704,7 +705,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   static_assert(NS >= 5, "the step reads three resident tiles and keeps at least one in flight");
 #pragma unroll
   for (int j = 0; j < NS - 3; ++j) issue(j);
-  loads_landed_but<(NS - 4) * PER_ISSUE>();
+  loads_landed_but<(NS - 4) * TI>();
   __syncthreads();
   // The step's products: product 2h is accumulation h (A^T from transposing
   // reads of the tile at abase: 16 keys c = h / DT, dims 32 (h % DT) ..; B =
@@ -813,7 +814,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
     // role 0: dV^T += dO^T P and S = Q K^T of the next tile;
     // role 1: dK^T += Q^T dS and dP = dO V^T of the next tile
     run(QG[SA], mf, QG[SS]);
-    loads_landed_but<(NS - 4) * PER_ISSUE>();
+    loads_landed_but<(NS - 4) * TI>();
     __syncthreads();
   };
   using std::integral_constant;
@@ -821,7 +822,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   if (kw0 >= S) {  // a slice without keys: only its waves' share of the loads
     for (; t <= n_it + 1; ++t) {
       issue((t + NS - 3) % NS);
-      loads_landed_but<(NS - 4) * PER_ISSUE>();
+      loads_landed_but<(NS - 4) * TI>();
       __syncthreads();
     }
     loads_landed_but<0>();
