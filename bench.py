@@ -325,7 +325,7 @@ def make_workload(name: str, dev: torch.device, head_dim: int = 128) -> Workload
                         "qk_norm_rope_bwd_kernel", bwd_bytes, launch,
                         {"batch": B, "q_heads": HQ, "kv_heads": HKV, "seq": S, "head_dim": D, "cos_batch": 1,
                          "eps": 1e-6, "dtype": "bf16"}, cpu, torch_step,
-                        launch_kernels=("qk_norm_rope_bwd_kernel", "column_sum_stage", "column_sum_final"))
+                        launch_kernels=("qk_norm_rope_bwd_kernel", "column_sum"))
 
     if name == "c4":
         rows, cols = 65536, 8192
@@ -375,7 +375,7 @@ def make_workload(name: str, dev: torch.device, head_dim: int = 128) -> Workload
         return Workload("c4", "RMSNorm fwd+bwd bf16 x, dy [65536, 8192]", "bf16", "TB/s", fwd_bytes + bwd_bytes,
                         step, "rmsnorm_bwd_vec", bwd_bytes, launch,
                         {"rows": rows, "cols": cols, "eps": 1e-6, "dtype": "bf16"}, cpu, torch_step,
-                        launch_kernels=("rmsnorm_bwd_vec", "column_sum_stage", "column_sum_final"))
+                        launch_kernels=("rmsnorm_bwd_vec", "column_sum"))
 
     if name == "add_rmsnorm":
         # not a BASELINE config: the next op on the norm path (residual add + RMSNorm) at C4's shape
@@ -426,7 +426,7 @@ def make_workload(name: str, dev: torch.device, head_dim: int = 128) -> Workload
         return Workload("add_rmsnorm", "add_rms_norm fwd+bwd bf16 x, residual, dy, ds [65536, 8192], offset 1",
                         "bf16", "TB/s", fwd_bytes + bwd_bytes, step, "rmsnorm_bwd_vec", bwd_bytes, launch,
                         {"rows": rows, "cols": cols, "eps": 1e-6, "offset": 1.0, "dtype": "bf16"}, cpu, torch_step,
-                        launch_kernels=("rmsnorm_bwd_vec", "column_sum_stage", "column_sum_final"))
+                        launch_kernels=("rmsnorm_bwd_vec", "column_sum"))
 
     if name in ("attn_bwd", "attn_bwd_f32"):
         # not a BASELINE config: attention forward + backward at C5's shape (causal), bf16 or, for

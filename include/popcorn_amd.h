@@ -105,11 +105,11 @@ int pk_rmsnorm_bwd(const void* x, const void* w, const float* rstd, const void* 
 
 /*
  * pk_rmsnorm_bwd without a workspace argument and without any allocation:
- * the dw / dbias partial rows and the column-sum stage live in a fixed
+ * the dw / dbias partial rows live in a fixed
  * file-scope device array of 96 MiB (100,663,296 bytes), which every GPU the
  * library runs on holds until the process ends. The kernels, grid and
  * summation order are pk_rmsnorm_bwd's, so the results are identical bit for
- * bit. A shape whose partial rows and stage do not fit the array (their size
+ * bit. A shape whose partial rows do not fit the array (their size
  * is at most pk_rmsnorm_bwd_workspace) is refused with PK_ERR_UNSUPPORTED
  * before any launch, and before the pointers are checked, so the limit can be
  * probed with null pointers: measured on MI355X, 65,536 rows of 8192 columns fit
