@@ -392,11 +392,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
 
   // ---- fast sweep: fixed max; each step exponentiates S(t), then runs the
   // products of O += V(t)^T P(t)^T and S(t+1) over the same S registers
-  // Key group k of NG takes tiles k, k + NG, ...; all run the same number of
-  // steps, tiles past the end being masked whole (their V is the last tile's).
-  // Every group takes its reference max from tile 0, so their sums add up
-  // without rescaling.
+  // Key group k of NG takes tiles k, k + NG, ...: its `own` steps, one fewer
+  // than group 0's where the tiles run out before it (there it only keeps the
+  // barriers: a step on any tile but its own, though masked whole, would
+  // multiply that tile's V by zero, and an Inf in it is a NaN then). Every group
+  // takes its reference max from tile 0, so their sums add up without rescaling.
   const int n_steps = NG == 1 ? n_tiles : (n_tiles + NG - 1) / NG;
+  const int own = NG == 1 ? n_tiles : (n_tiles - kgrp + NG - 1) / NG;
   auto tile_of = [&](int j) { return NG == 1 ? j : kgrp + NG * j; };
   clear();
   dma_k(NG == 1 ? 0 : min(tile_of(0), n_tiles), 0);
@@ -482,12 +484,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NG * NT, NG * NT), amdgpu_
     }
     return;
   }
-  for (int t = 0;;) {
+  for (int t = 0; NG == 1 || t < own;) {
     step(t, std::integral_constant<int, 0>{});
-    if (++t >= n_steps) break;
+    if (++t >= own) break;
     step(t, std::integral_constant<int, 1>{});
-    if (++t >= n_steps) break;
+    if (++t >= own) break;
   }
+  if (NG > 1 && own < n_steps) __syncthreads();
   if constexpr (NG > 1) {
     // groups 1 .. NG - 1 leave O^T and l in LDS (the tiles are done with: the
     // last step ended with a barrier); group 0 adds them in order

@@ -122,3 +122,24 @@ def test_attn_nonfinite_key_and_value(causal, dtype):
         ref = R.attn(q, k, v, causal)
         mine = impls.attn(q.to(DEV), k.to(DEV), v.to(DEV), causal)
     _same_pattern(mine, ref, f"attn {dtype} causal={causal}")
+
+
+# rows of 51 or 50 key tiles, so that one key group or more of a split block has a step less than the others
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("s,d", [(1620, 32), (1620, 64), (1600, 96), (1600, 128), (1620, 192), (1620, 256)])
+def test_attn_infinite_value_in_the_last_tile_of_split_keys(s, d, causal):
+    """An Inf in the value row of a key of the last tile: the queries that see the key get the Inf in that
+    dim, as without the split (a batch that fills the grid); every other dim is untouched."""
+    key, dim = s - 10, 7
+    q, k, v = (seeded((1, s, h, d), 40 + i, torch.bfloat16) for i, h in enumerate((4, 2, 2)))
+    v = _plant(v, [((0, key, 1, dim), INF)])
+    q, k, v = (t.to(DEV) for t in (q, k, v))
+    copies = 4096 // (4 * (s // 128)) + 1  # more than two blocks per CU at any row group
+    with torch.no_grad():
+        for mine, full in ((impls.attn(q, k, v, causal), impls.attn(*(t.repeat(copies, 1, 1, 1) for t in (q, k, v)), causal)),
+                           (impls.attn_with_lse(q, k, v, causal)[0], None)):
+            assert mine[0, key if causal else 0:, 2:, dim].isposinf().all()
+            assert mine[..., :dim].isfinite().all() and mine[..., dim + 1:].isfinite().all()
+            assert mine[:, :, :2].isfinite().all()
+            if full is not None:
+                _same_pattern(mine, full[:1].cpu(), f"attn d={d} causal={causal}")
