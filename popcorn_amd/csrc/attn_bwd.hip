@@ -699,9 +699,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   // Step t reads tiles t - 2 .. t (the stage ring holds NS). It issues tile
   // t + NS - 3 into the stage of tile t - 3, last read in step t - 1, and
   // ends once tile t + 1 has landed, leaving NS - 4 tiles in flight. Before
-  // the first tile and after the last the wave's tile indices are clamped into
-  // the range (those stages hold landed, finite data) and its accumulation
-  // factors are zero, so the edge steps run the same products to no effect.
+  // tile 0 is scored a wave has nothing to accumulate, and after the last tile
+  // role 0 only keeps the barrier of role 1's last step: products with zero
+  // factors in their place would turn an Inf of the tile they read into a NaN.
   static_assert(NS >= 5, "the step reads three resident tiles and keeps at least one in flight");
 #pragma unroll
   for (int j = 0; j < NS - 3; ++j) issue(j);
@@ -749,15 +749,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   // (tau - 1) % NS and tau % NS, so the steps are unrolled over the NS stage
   // phases of tau and every fragment address is a lane register plus an
   // immediate. Past the last tile those stages hold landed copies of it (the
-  // cursor issues the last tile again), the same data the clamped indices
-  // name. The first steps (tau <= 0, before tile 0 is scored) read stage 0.
+  // cursor issues the last tile again), whose score block nobody uses.
   auto body = [&](int t, auto a_stage, auto s_stage) {
     constexpr int SA = decltype(a_stage)::value, SS = decltype(s_stage)::value;
     issue((t + NS - 3) % NS);
     const int u = t - 1 - role;
-    const bool live = u >= 0 && u < n_it;
     Frag mf[2];
-    if (live) {
+    {
       const int st = SA;  // u % NS
       float rv[16];  // the tile rows' lse2 (role 0) or D (role 1)
       rows16(RV[st][role], rv);
@@ -805,11 +803,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
           }
         }
       }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) mf[c][j] = (T)0.f;
     }
     // role 0: dV^T += dO^T P and S = Q K^T of the next tile;
     // role 1: dK^T += Q^T dS and dP = dO V^T of the next tile
@@ -828,22 +821,35 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
     loads_landed_but<0>();
     return;  // past the block's last barrier
   }
-  for (; t <= role; ++t) body(t, integral_constant<int, 0>{}, integral_constant<int, 0>{});  // tau <= 0
+  for (; t <= role; ++t) {  // tau <= 0: tile 0, in stage 0, is scored
+    issue((t + NS - 3) % NS);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sres[r] = 0.f;
+#pragma unroll
+    for (int h = 0; h < KS; ++h) sres = Mma<T>::run(*reinterpret_cast<const Frag*>(QG[0] + a_lane[h]), bf[h], sres);
+    loads_landed_but<(NS - 4) * TI>();
+    __syncthreads();
+  }
+  // The compiler is not to know that the accumulators start as zeros: it then
+  // carries them through the loop as single registers, and spills 290 of them.
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) asm volatile("" : "+v"(acc[dt]));
   static_assert(NS == 6, "the step loop is unrolled over six stage phases");
   for (;;) {  // tau = t - role >= 1, phase tau % NS = 1, 2, ..., 5, 0
-    if (t > n_it + 1) break;
+    if (t > n_it + role) break;
     body(t++, integral_constant<int, 0>{}, integral_constant<int, 1>{});
-    if (t > n_it + 1) break;
+    if (t > n_it + role) break;
     body(t++, integral_constant<int, 1>{}, integral_constant<int, 2>{});
-    if (t > n_it + 1) break;
+    if (t > n_it + role) break;
     body(t++, integral_constant<int, 2>{}, integral_constant<int, 3>{});
-    if (t > n_it + 1) break;
+    if (t > n_it + role) break;
     body(t++, integral_constant<int, 3>{}, integral_constant<int, 4>{});
-    if (t > n_it + 1) break;
+    if (t > n_it + role) break;
     body(t++, integral_constant<int, 4>{}, integral_constant<int, 5>{});
-    if (t > n_it + 1) break;
+    if (t > n_it + role) break;
     body(t++, integral_constant<int, 5>{}, integral_constant<int, 0>{});
   }
+  if (role == 0) __syncthreads();
   loads_landed_but<0>();  // tiles issued past the end, before the block's LDS is released
 
   if (key_ok) {

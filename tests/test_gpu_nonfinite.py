@@ -143,3 +143,28 @@ def test_attn_infinite_value_in_the_last_tile_of_split_keys(s, d, causal):
             assert mine[:, :, :2].isfinite().all()
             if full is not None:
                 _same_pattern(mine, full[:1].cpu(), f"attn d={d} causal={causal}")
+
+
+# dk/dv grids whose query tiles are split into runs of 32 tiles (2 or 4 of them without the mask): rows in the
+# first and in the last tile of a run, and of the whole call
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("row", [3, 1023, 1029, 2047, 2048, 4090])
+@pytest.mark.parametrize("d", [64, 128])
+def test_attn_infinite_cotangent_at_the_edges_of_split_queries(d, row, causal):
+    """An Inf in the cotangent of one row: dv of every key the row sees gets the Inf in that dim, no other dim of
+    dv is touched, and the gradients hold their Inf and NaN where those of an unsplit grid do."""
+    s, dim = 4096, 7
+    q, k, v, do = (seeded((1, s, 1, d), 50 + i, torch.bfloat16).to(DEV) for i in range(4))
+    do[0, row, 0, dim] = INF
+
+    def grads(*ts):
+        leaves = [t.clone().requires_grad_() for t in ts[:3]]
+        return torch.autograd.grad(impls.attn(*leaves, causal), leaves, ts[3])
+
+    mine = grads(q, k, v, do)
+    full = grads(*(t.repeat(17, 1, 1, 1) for t in (q, k, v, do)))  # two blocks of 128 keys per CU
+    dv = mine[2][0, :, 0]
+    assert dv[: row + 1 if causal else s, dim].isposinf().all()
+    assert dv[:, :dim].isfinite().all() and dv[:, dim + 1:].isfinite().all()
+    for name, a, b in zip(("dq", "dk", "dv"), mine, full):
+        _same_pattern(a, b[:1].cpu(), f"{name} d={d} row={row} causal={causal}")
