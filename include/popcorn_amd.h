@@ -127,6 +127,8 @@ int pk_rmsnorm_bwd_noalloc(const void* x, const void* w, const float* rstd, cons
  *   s = round(x + residual); r = 1/sqrt(mean(s^2) + eps);
  *   y = round(round(s*r) * round(w + offset)).
  * Writes y and s (the new residual stream); rstd (fp32 [rows]) may be NULL.
+ * s may be x or residual (in place), at any width and alignment; outputs
+ * overlap nothing else.
  * x, residual and s have `dtype`; w and y have `w_dtype`: `dtype`, or fp32
  * with a 16-bit `dtype` (torch's promotion: w + offset stays fp32 and the
  * product with the rounded 16-bit row is an fp32 y). Replaces: reference

@@ -128,7 +128,9 @@ template <typename T, typename W, bool BIAS> __device__ __forceinline__ W fwd_el
   return from_f32<W>(y);
 }
 
-// One row per TPR lanes, RPB = NTB / TPR rows per block.
+// One row per TPR lanes, RPB = NTB / TPR rows per block. s_out may be x or res:
+// a pack of its own (ALN) is stored once it is loaded, but packs that overlap
+// only after the row's reduction, when every lane has the elements it reads.
 template <typename T, typename W, int NTB, int TPR, int VPT, int MODE, bool ALN>
 __global__ __launch_bounds__(NTB) void rmsnorm_fwd_vec(const T* __restrict__ x, const W* __restrict__ w,
                                                        const W* __restrict__ bias, const T* __restrict__ res,
@@ -157,7 +159,7 @@ __global__ __launch_bounds__(NTB) void rmsnorm_fwd_vec(const T* __restrict__ x, 
       xv[k] = ld16_stream_at<ALN>(xr + at.start);
       if constexpr (MODE == kAdd) {
         add_residual(xv[k], ld16_stream_at<ALN>(res + row * cols + at.start));
-        st16_stream_at<ALN>(s_out + row * cols + at.start, xv[k]);
+        if constexpr (ALN) st16_stream_at<ALN>(s_out + row * cols + at.start, xv[k]);
       }
 #pragma unroll
       for (int j = 0; j < P; ++j) {
@@ -177,6 +179,12 @@ __global__ __launch_bounds__(NTB) void rmsnorm_fwd_vec(const T* __restrict__ x, 
     const int v = fwd_pack<NTB, TPR, VPT>(lane, k);
     if (v < nvec) {
       const PackAt<ALN, P> at(v, nvec, cols);
+      if constexpr (MODE == kAdd && !ALN) {
+        u32x4 bits = *reinterpret_cast<const u32x4*>(&xv[k]);
+        asm volatile("" : "+v"(bits) : "v"(r));  // not before r, for the compiler either
+        *reinterpret_cast<u32x4*>(&xv[k]) = bits;
+        st16_stream_at<ALN>(s_out + row * cols + at.start, xv[k]);
+      }
       Lane<W, P> wv = ld_lane_at<ALN, W, P>(w + at.start);
       if constexpr (MODE == kAdd) wv = offset_weight(wv, offset);
       Lane<W, P> bv;

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import reference as O
-from popcorn_amd import impls
+from popcorn_amd import _lib, impls
 from popcorn_amd.compat import references as R
 from tests._parity import gauge_ok, seeded
 
@@ -89,3 +89,27 @@ def test_ragged_residual_add(dtype, wdtype, cols):
     gauge_ok(y, y64.detach().numpy(), ref[0], wdtype, "y")
     for name, g, t, q in zip(("dx", "dr", "dw"), got, g64, gref):
         gauge_ok(g, t.numpy(), q, g.dtype, f"{name} cols {cols}")
+
+
+# one wave to a row and a block to a row, the last pack overlapping by one element and by all but one, whole
+# packs, rows narrower than a pack and wider than the row kernels take
+@pytest.mark.parametrize("dtype,cols", [
+    (torch.float32, c) for c in (3, 5, 7, 1024, 1025, 1537, 4099, 70001)] + [
+    (torch.bfloat16, c) for c in (9, 15, 2041, 2049, 4097, 8199, 4096)] + [(torch.float16, 1001)], ids=str)
+@pytest.mark.parametrize("into", ["x", "residual"])
+def test_add_rms_norm_into_its_own_residual_stream(dtype, cols, into):
+    """s written over x or over residual: y, s and rstd are those of a call with buffers of their own."""
+    rows, lib = 67, _lib.load()
+    x, r, w = seeded((rows, cols), 1, dtype).to(DEV), seeded((rows, cols), 2, dtype).to(DEV), seeded((cols,), 3, dtype).to(DEV)
+
+    def call(x, r, s):
+        y, rstd = torch.empty_like(x), torch.empty(rows, device=DEV)
+        _lib.check(lib.pk_add_rmsnorm_fwd(x.data_ptr(), r.data_ptr(), w.data_ptr(), y.data_ptr(), s.data_ptr(),
+                                          rstd.data_ptr(), rows, cols, 1e-6, 1.0, _lib.dtype_code(dtype),
+                                          _lib.dtype_code(dtype), _lib.stream_handle(x.device)))
+        return y, s, rstd
+
+    want = call(x, r, torch.empty_like(x))
+    mine = {"x": x.clone(), "residual": r.clone()}
+    for a, b in zip(call(mine["x"], mine["residual"], mine[into]), want):
+        assert torch.equal(a, b)
