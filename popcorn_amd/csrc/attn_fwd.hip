@@ -608,23 +608,38 @@ int launch_groups(AttnArgs a, bool causal, hipStream_t s) {
 // 4.5 us once (D 128; the wider block's start and the sum over the groups), and
 // its groups share every barrier. So it is for grids that cannot fill the CUs
 // with blocks of one group, and rows long enough to earn the cost back. Measured
-// (us, one group -> split; bf16):
-//   one block per CU:  D 128 causal, 256 tiles 167 -> 102, 32 tiles 26.1 -> 24.3, 16 tiles 15.8 -> 17.1;
-//                      full, 32 tiles 25.0 -> 25.0; D 64, causal 64 tiles 31.0 -> 22.4, 16 tiles
-//                      11.2 -> 11.0, full 33 tiles 17.4 -> 15.5
-//   two, causal:       D 128, 512 tiles 372 -> 261, 64 tiles 53.2 -> 49.4; D 96, 64 tiles 42.1 -> 41.1;
-//                      D 192, 128 tiles 132 -> 113; D 256, 64 tiles 84.1 -> 83.0; D 64, 64 tiles 35.3 -> 38.4
-//   two, full:         D 128, 64 tiles 66.7 -> 79.2 (the blocks are equally long and two share a CU)
-//   four:              D 128, 128 tiles causal 133 -> 155
-// A call that keeps its log-sum-exp for a backward splits only from rows on
-// where that backward's dq kernel does: below, a sequence then has the same
-// gradients, to a unit of its type, alone and in a batch that fills the grid.
+// (us, one group -> split; bf16; 4 q heads to a kv head, or as said):
+//   one block per CU, causal, at 20, 24, 28, 32 and 48 tiles:
+//     D 64   12.6 -> 12.2, 14.4 -> 13.2, 16.0 -> 14.3, 17.5 -> 15.3, 23.8 -> 18.8 (D 32 alike; full: 20 alike,
+//            24 14.9 -> 14.3, 48 24.0 -> 20.2)
+//     D 128  17.8 -> 18.2, 22.3 -> 20.1, 26.7 -> 22.1, 24.5 -> 22.7, 39.8 -> 29.0 (D 96 gains from 24 on)
+//     D 192  22.3 -> 22.7, 25.8 -> 25.6, 28.0 -> 27.2, 30.3 -> 29.3, 39.9 -> 37.2
+//     D 256  27.3 -> 28.4, 31.8 -> 31.9, 33.8 -> 33.5, 37.1 -> 36.0, 48.9 -> 46.0
+//   one block per CU, full, at 32, 40 and 48 tiles: D 128 26.0 -> 25.0, 29.8 -> 27.7, 40.5 -> 31.7;
+//     one head to a kv head D 96 22.9 -> 21.4, 27.0 -> 29.3, 31.3 -> 29.9, D 256 41.7 -> 42.3, 51.9 -> 51.7, 57.6 -> 56.7
+//   two, causal, at 64, 72, 80, 96 and 128 tiles:
+//     D 128  50.9 -> 47.2, 59.1 -> 53.0, 63.9 -> 53.2, 75.3 -> 63.3, 99.4 -> 77.1; one head to a kv head (at 64
+//            tiles a multiple of 8 groups, which dense_item runs one after another) 54.1 -> 60.1, 59.4 -> 54.3,
+//            67.8 -> 61.2, 78.7 -> 70.0, 99.0 -> 80.9
+//     D 256  76.9 -> 79.8, 85.1 -> 89.9, 90.8 -> 89.5, 106 -> 106, 143 -> 136 (112 tiles, two heads 127 -> 128)
+//     D 64   31.9 -> 31.2, one head to a kv head 32.4 -> 38.8; 192 tiles 81.1 -> 53.3
+//   one and a half, causal, at 64, 72 and 96 tiles: D 256 69.7 -> 65.0, 75.7 -> 67.2, 97.7 -> 86.1; one head to a kv head
+//     71.5 -> 80.5, 83.0 -> 74.4, 98.3 -> 87.1
+//   two, full:  D 128, 64 tiles 64.1 -> 76.8 (the blocks are equally long and two share a CU)
+//   four:       D 128, 128 tiles causal 133 -> 155
+// Calls that keep their log-sum-exp for a backward split from 32 (D <= 64) or 48
+// tiles on at one block per CU: O enters that backward through D = rowsum(dO O),
+// and on shorter rows a sequence's O and gradients are then the same alone and
+// in a batch that fills the grid. (The backward's dq has lines of its own, split_dq.)
 template <int D> bool split_keys(const AttnArgs& a, bool causal) {
   const int tiles = (a.S + BN - 1) / BN;
   const int64_t blocks = fwd_blocks(a), cus = cu_count();
   const bool alone = a.lse == nullptr;
   if (blocks <= cus) return tiles >= (D <= 64 ? (alone ? 24 : 32) : (alone && causal ? 28 : 48));
-  return blocks <= 2 * cus && causal && tiles >= (D <= 64 ? 192 : 64);
+  if (!causal || blocks > 2 * cus) return false;
+  if (D <= 64) return tiles >= 192;
+  if (D > 128 && 2 * blocks > 3 * cus) return tiles >= 128;
+  return tiles >= (a.gp > 1 ? 64 : 72);
 }
 
 template <typename T, int D, int KS>

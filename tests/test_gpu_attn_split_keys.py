@@ -31,8 +31,8 @@ def _inputs(s, hq, hkv, d, dtype, seed):
             seeded((1, s, hkv, d), seed + 2, dtype))
 
 
-# tiles of 32 keys around multiples of the group count (2, 3 and 4 groups), a last tile of one key, and
-# rows of every layout; the causal 2049 has two blocks per CU only where the group count below gives it
+# one block per CU: tiles of 32 keys around multiples of the group count (2, 3 and 4 groups), a last tile of one
+# key, and rows of every layout
 @pytest.mark.parametrize("s,hq,hkv,d,dtype,causal", [
     (1023, 4, 1, 64, torch.bfloat16, True),
     (1025, 6, 2, 64, torch.float16, False),
@@ -45,10 +45,9 @@ def _inputs(s, hq, hkv, d, dtype, seed):
 ], ids=str)
 def test_split_rows_match_the_unsplit_kernel(s, hq, hkv, d, dtype, causal):
     q, k, v = (t.to(DEV) for t in _inputs(s, hq, hkv, d, dtype, 3 * d))
-    copies = 4096 // (hq * (s // 128)) + 1  # more than two blocks per CU at any row group
     with torch.no_grad():
         o, lse = impls.attn_with_lse(q, k, v, causal)
-        wide, wide_lse = impls.attn_with_lse(*(t.repeat(copies, 1, 1, 1) for t in (q, k, v)), causal)
+        wide, wide_lse = impls.attn_with_lse(*(t.repeat(_copies(s, hq), 1, 1, 1) for t in (q, k, v)), causal)
     tiles = -(-s // 32)
     bound = v.float().abs().max().item() * (2 * tiles * 2.0**-24 + ULP[dtype])
     assert (o.float() - wide[:1].float()).abs().max().item() <= bound
@@ -60,6 +59,56 @@ def test_split_rows_match_the_unsplit_kernel(s, hq, hkv, d, dtype, causal):
         o64, lse64 = O.attention_rows(qh, kh, vh, rows, causal)
         assert np.abs(o[0, rows, h].double().cpu().numpy() - o64).max() < 2e-2 * max(1.0, np.abs(o64).max())
         np.testing.assert_allclose(lse[0, h, rows].double().cpu().numpy(), lse64, rtol=0, atol=1e-3)
+
+
+def _copies(s, hq):
+    return 4096 // (hq * (s // 128)) + 1  # more than two blocks per CU at any row group
+
+
+# one block per CU, of 24 to 31 (up to 64 dims) and 28 to 47 key tiles: split where no log-sum-exp is kept
+@pytest.mark.parametrize("s,hq,hkv,d,dtype,causal", [
+    (768, 4, 1, 64, torch.bfloat16, True),
+    (991, 6, 2, 32, torch.float16, False),
+    (896, 4, 4, 128, torch.bfloat16, True),
+    (1021, 32, 8, 128, torch.bfloat16, True),
+    (1500, 2, 1, 192, torch.bfloat16, True),
+    (900, 4, 2, 256, torch.float16, True),
+], ids=str)
+def test_split_without_a_log_sum_exp(s, hq, hkv, d, dtype, causal):
+    """No more than the order of the sum over tiles differs from an unsplit grid, and it does differ (the call
+    was split); with a log-sum-exp, as a call that is recorded for a backward has it, not even that."""
+    q, k, v = (t.to(DEV) for t in _inputs(s, hq, hkv, d, dtype, 2 * d))
+    many = [t.repeat(_copies(s, hq), 1, 1, 1) for t in (q, k, v)]
+    with torch.no_grad():
+        o, wide = impls.attn(q, k, v, causal), impls.attn(*many, causal)[:1]
+        kept = impls.attn_with_lse(q, k, v, causal)[0]
+    recorded = impls.attn(q.clone().requires_grad_(), k, v, causal).detach()
+    bound = v.float().abs().max().item() * (2 * -(-s // 32) * 2.0**-24 + ULP[dtype])
+    assert (o.float() - wide.float()).abs().max().item() <= bound
+    assert not torch.equal(o, wide)
+    assert torch.equal(kept, wide) and torch.equal(recorded, wide)
+
+
+# causal grids of 257 to 512 blocks (256 CUs): on either side of the lines of split_keys
+@pytest.mark.parametrize("s,hq,hkv,d,split", [
+    (2048, 32, 32, 128, False),  # one head to a kv head: from 72 tiles on
+    (2304, 26, 26, 128, True),
+    (2048, 32, 8, 96, True),  # four heads: from 64
+    (2048, 32, 32, 256, False),  # wide rows: up to 384 blocks as above, past them from 128 tiles on
+    (2310, 17, 17, 192, True),
+    (3072, 21, 21, 192, False),
+    (4096, 16, 16, 256, True),
+    (6100, 8, 8, 64, False),  # up to 64 dims: from 192
+    (6150, 8, 8, 64, True),
+], ids=str)
+def test_split_at_two_blocks_per_cu(s, hq, hkv, d, split):
+    q, k, v = (t.to(DEV) for t in _inputs(s, hq, hkv, d, torch.bfloat16, d + 1))
+    with torch.no_grad():
+        o = impls.attn(q, k, v, True)
+        wide = impls.attn(*(t.repeat(_copies(s, hq), 1, 1, 1) for t in (q, k, v)), True)[:1]
+    bound = v.float().abs().max().item() * (2 * -(-s // 32) * 2.0**-24 + ULP[torch.bfloat16])
+    assert (o.float() - wide.float()).abs().max().item() <= bound
+    assert torch.equal(o, wide) is not split
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
