@@ -939,14 +939,21 @@ int64_t key_grid(BwdArgs& a) {
 #include "attn_bwd_f32.h"
 #include "attn_bwd_wide.h"
 
-// Whether the dq kernel splits its keys, by the rule of the forward (attn_fwd.hip,
-// split_keys). One pk_attn_bwd call, us, one group -> split (bf16, causal):
-//   one block per CU:  D 128, 256 tiles 444 -> 401, 64 tiles 118 -> 111, 32 tiles 90.0 -> 85.3 (one unit
-//                      of dq is not worth that: see split_keys), 16 tiles 55.2 -> 54.5;
-//                      D 64, 64 tiles 84.5 -> 78.4; full, 32 tiles 91.2 -> 91.2
-//   two:               D 128, 512 tiles 1005 -> 964, 128 tiles 295 -> 274, 64 tiles 173.1 -> 173.9;
-//                      D 64, 512 tiles 684 -> 611, 64 tiles 105 -> 111; full, 64 tiles 270 -> 284
-//   four:              D 128, 128 tiles 508 -> 530
+// Whether the dq kernel splits its keys: as in the forward (attn_fwd.hip, split_keys),
+// for grids that cannot fill the CUs and rows long enough, with lines of its own:
+// the kernel without the split has two tiles in flight already and gains less.
+// One pk_attn_bwd call, us, one group -> split (bf16; 4 q heads to a kv head, or as said):
+//   one block per CU, causal:  D 64, 20 tiles 45.3 -> 45.1, 32 59.0 -> 56.5, 48 75.9 -> 69.5; D 128, 24 70.9 -> 70.7,
+//                              32 84.0 -> 82.4, 48 108 -> 103, 256 351 -> 309; D 96, 48 94.1 -> 90.4
+//   one, full:                 D 64, 32 61.6 -> 59.4, 48 79.4 -> 73.9; D 128, 32 89.0 -> 86.9, 48 114 -> 111; one head to
+//                              a kv head D 96, 40 81.4 -> 81.9, 48 94.1 -> 93.3
+//   two, causal:               D 64, 96 138 -> 132, 192 207 -> 175, one head to a kv head 64 96.7 -> 108, 192 245 -> 219;
+//                              D 128, 64 167 -> 168, 96 244 -> 241, 128 292 -> 283, one head to a kv head 64 155 -> 175,
+//                              96 268 -> 270, 128 267 -> 263
+//   two, full:                 D 64, 192 329 -> 348; D 128, 64 258 -> 270, 256 858 -> 899
+//   four:                      D 128, causal, 128 tiles 508 -> 530
+// (Below these lines a sequence's dq has the same bits alone and in a batch that
+// fills the grid, which a few per cent were not worth.)
 template <int D> bool split_dq(const BwdArgs& a, int64_t blocks, bool causal) {
   const int tiles = (a.S + BN - 1) / BN;
   const int64_t cus = cu_count();

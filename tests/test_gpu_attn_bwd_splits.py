@@ -32,19 +32,24 @@ def _grads(q, k, v, do, causal):
     return torch.autograd.grad(impls.attn(*leaves, causal), leaves, do)
 
 
-# 2 and 4 runs of query tiles, ragged ends, groups that split their heads too, every row layout
-@pytest.mark.parametrize("s,hq,hkv,d,dtype,causal", [
-    (2048, 4, 4, 64, torch.bfloat16, True),
-    (2049, 2, 1, 128, torch.float16, True),
-    (4097, 1, 1, 128, torch.bfloat16, True),
-    (4100, 2, 2, 32, torch.bfloat16, False),
-    (2500, 6, 2, 80, torch.bfloat16, True),
-    (2080, 3, 3, 96, torch.float16, False),
+# 2 and 4 runs of query tiles (at these sizes the same number with the mask and without), ragged ends, groups that
+# split their heads too, every row layout; `heads` and `runs` are what 256 CUs get. The last two have a dq grid of
+# more than one and up to two blocks per CU, split from 96 and, up to 64 dims, 192 key tiles on
+@pytest.mark.parametrize("s,hq,hkv,d,dtype,causal,heads,runs", [
+    (2048, 4, 4, 64, torch.bfloat16, True, 1, 2),
+    (2049, 2, 1, 128, torch.float16, True, 2, 2),
+    (4097, 1, 1, 128, torch.bfloat16, True, 1, 4),
+    (4100, 2, 2, 32, torch.bfloat16, False, 1, 4),
+    (2500, 6, 2, 80, torch.bfloat16, True, 3, 2),
+    (2080, 3, 3, 96, torch.float16, False, 1, 2),
+    (3100, 16, 16, 128, torch.bfloat16, True, 1, 2),
+    (6150, 8, 8, 64, torch.bfloat16, True, 1, 2),
 ], ids=str)
-def test_split_grids_match_a_full_one(s, hq, hkv, d, dtype, causal):
+def test_split_grids_match_a_full_one(s, hq, hkv, d, dtype, causal, heads, runs):
     q, k, v, do = (seeded((1, s, h, d), 7 + i, dtype).to(DEV) for i, h in enumerate((hq, hkv, hkv, hq)))
     lse = -(-2 * hq * s * 4 // 256) * 256
-    assert _lib.load().pk_attn_bwd_workspace(1, s, hq, hkv, d) > lse  # the query tiles are split
+    partials = heads * runs * 2 * s * hkv * (64 if d <= 64 else 128) * 4
+    assert _lib.load().pk_attn_bwd_workspace(1, s, hq, hkv, d) == lse + partials
     copies = 512 // (hkv * (s // 128)) + 1
     got = _grads(q, k, v, do, causal)
     want = _grads(*(t.repeat(copies, 1, 1, 1) for t in (q, k, v, do)), causal)
