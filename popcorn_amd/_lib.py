@@ -117,11 +117,13 @@ def native():
         return _ThroughPython()
     load()
     try:
+        from torch.utils._device import DeviceContext
+
         from popcorn_amd import _native as module
 
         if module.ABI_VERSION != ABI_VERSION or module.TORCH_VERSION != torch.__version__:
             raise ImportError(f"built for ABI {module.ABI_VERSION} and torch {module.TORCH_VERSION}")
-        module.set_error(KernelError)
+        module.set_types(KernelError, DeviceContext)
         _native = module
     except ImportError as e:
         warnings.warn(f"popcorn_amd: {NATIVE.name} cannot be used ({e}); calls go through Python. Rebuild with "

@@ -8,12 +8,13 @@
 // the host in Python and ctypes.
 //
 // For any other call a function returns NotImplemented before it does anything,
-// and impls.py takes it: tensor subclasses and calls under tracing, dispatch
-// modes or function transforms, layouts that need a copy, empty tensors, and
-// every call that has to be refused. So what is accepted and how errors read is
+// and impls.py takes it: tensor subclasses and calls under tracing, dispatch or
+// function modes or function transforms, layouts that need a copy, empty tensors,
+// and every call that has to be refused. So what is accepted and how errors read is
 // said there, and here only what the fast path covers.
 #include <Python.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TracerMode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
@@ -23,6 +24,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -42,7 +44,8 @@ using torch::autograd::AutogradContext;
 using torch::autograd::Function;
 using torch::autograd::variable_list;
 
-PyObject* kernel_error = nullptr;  // popcorn_amd._lib.KernelError
+PyObject* kernel_error = nullptr;    // popcorn_amd._lib.KernelError
+PyObject* device_context = nullptr;  // torch.utils._device.DeviceContext
 
 // Raises KernelError, from any thread.
 void check(int status) {
@@ -72,9 +75,21 @@ bool plain(const Tensor& t) {
          is_float(t.scalar_type()) && t.numel() > 0 && !t._fw_grad(0).defined();
 }
 
+// Whether a torch function mode is active that could look at the torch calls
+// inside one of these. The one behind torch.set_default_device and `with
+// torch.device(..)` only gives a device to calls that name none.
+bool function_mode() {
+  if (!at::impl::torch_function_mode_enabled()) return false;
+  for (int64_t i = 0; i < at::impl::PythonTorchFunctionTLS::stack_len(); ++i) {
+    const PyObject* mode = at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter());
+    if ((const PyObject*)Py_TYPE(mode) != device_context) return true;
+  }
+  return false;
+}
+
 // Calls some mode or transform means to see operator by operator.
 bool watched() {
-  return c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || function_mode() ||
          c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
          at::tracer::impl::is_dispatch_enabled();
 }
@@ -679,11 +694,14 @@ PyObject* py_attn_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// The library and torch this was compiled against, for the importer to compare, and the exception to raise.
-PyObject* py_set_error(PyObject*, PyObject* cls) {
-  Py_INCREF(cls);
-  Py_XDECREF(kernel_error);
-  kernel_error = cls;
+// The exception to raise, and torch's mode of a default device.
+PyObject* py_set_types(PyObject*, PyObject* args) {
+  PyObject *error, *context;
+  if (!PyArg_ParseTuple(args, "OO", &error, &context)) return nullptr;
+  Py_INCREF(error);
+  Py_INCREF(context);
+  Py_XSETREF(kernel_error, error);
+  Py_XSETREF(device_context, context);
   Py_RETURN_NONE;
 }
 
@@ -692,12 +710,13 @@ PyMethodDef methods[] = {
     PK_FAST("rms_norm", py_rms_norm),         PK_FAST("add_rms_norm", py_add_rms_norm), PK_FAST("swiglu", py_swiglu),
     PK_FAST("rotary_embedding", py_rotary),   PK_FAST("rope", py_rope),                 PK_FAST("qk_norm_rope", py_qk_norm_rope),
     PK_FAST("attn", py_attn),                 PK_FAST("attn_varlen", py_attn_varlen),
-    {"set_error", py_set_error, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
+    {"set_types", py_set_types, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "popcorn_amd._native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
+// With the library and torch this was compiled against, for the importer to compare.
 PyMODINIT_FUNC PyInit__native() {
   PyObject* m = PyModule_Create(&module);
   if (m != nullptr && (PyModule_AddIntConstant(m, "ABI_VERSION", PK_ABI_VERSION) < 0 ||

@@ -132,3 +132,75 @@ def test_layouts_that_need_a_copy_and_subclasses_are_left_to_python():
     assert native.rms_norm(x.as_subclass(type("Sub", (torch.Tensor,), {})), w, None, 1e-6) is NotImplemented
     assert native.attn(*(_t((1, 9, 2, 64))[..., :60] for _ in range(3)), False, None) is NotImplemented
     assert torch.equal(impls.rms_norm(x.t().contiguous().t(), w), impls.rms_norm(x, w))
+
+
+def test_a_torch_function_mode_sees_the_calls_inside():
+    """As it does through Python; the mode of a default device, which changes nothing here, does not matter."""
+
+    class Seen(torch.overrides.TorchFunctionMode):
+        names = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.names.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    x, w = _t((4, 64)), _t((64,))
+    want = impls.rms_norm(x, w)
+    with Seen():
+        assert torch.equal(impls.rms_norm(x, w), want)
+    assert "empty" in Seen.names
+    with torch.device("cpu"):
+        assert torch.equal(_lib.native().rms_norm(x, w, None, 1e-6), want)
+        with Seen():
+            assert _lib.native().rms_norm(x, w, None, 1e-6) is NotImplemented
+    assert torch.equal(_lib.native().rms_norm(x, w, None, 1e-6), want)
+
+
+def test_tangents_are_refused_as_before(through_python):
+    """Forward-mode AD: no op has a jvp, so a dual input is refused and not read past its tangent."""
+    fwad = torch.autograd.forward_ad
+    x, w = _t((4, 64)), _t((64,))
+    for switch in (lambda: None, through_python):
+        switch()
+        with fwad.dual_level():
+            dual = fwad.make_dual(x, torch.ones_like(x))
+            if switch is not through_python:
+                assert _lib.native().rms_norm(dual, w, None, 1e-6) is NotImplemented
+            with pytest.raises(NotImplementedError):
+                impls.rms_norm(dual.requires_grad_(), w)
+        assert torch.equal(impls.rms_norm(x, w), impls.rms_norm(x.clone(), w))
+
+
+def test_a_traced_call_stays_in_python(monkeypatch):
+    """Where the tracer is at work the native path is not offered the call at all."""
+
+    class Refuses:
+        def __getattr__(self, name):
+            raise AssertionError("the native path was offered a traced call")
+
+    x, w = _t((4, 64)), _t((64,))
+    want = impls.rms_norm(x, w)
+    monkeypatch.setattr(impls, "_compiling", lambda: True)
+    monkeypatch.setattr(_lib, "_native", Refuses())
+    assert torch.equal(impls.rms_norm(x, w), want)
+
+
+@pytest.mark.parametrize("name", ["rms_norm", "swiglu", "attn"])
+def test_calls_go_on_the_current_stream(name):
+    """Forward and backward on a stream of their own, after work there that the inputs wait for."""
+    call, *specs = CASES[name]
+    want = _run(call, _leaves(specs))
+    side = torch.cuda.Stream()
+    ready = _leaves(specs)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        held = torch.randn(4096, 4096, device=DEV)
+        for _ in range(20):
+            held = held @ held * 1e-4  # some milliseconds ahead of the copies
+        late = [torch.zeros_like(t) for t in ready]
+        for dst, src in zip(late, ready):
+            dst.copy_(src.detach())
+        got = _run(call, [t.requires_grad_() for t in late])
+    side.synchronize()
+    for a, b in zip(got[0] + list(got[1]), want[0] + list(want[1])):
+        assert torch.equal(a, b)
