@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import sysconfig
 import threading
 import warnings
 from pathlib import Path
@@ -91,7 +92,7 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         return lib
 
 
-NATIVE = LIBRARY.with_name("_native.so")
+NATIVE = LIBRARY.with_name(f"_native{sysconfig.get_config_var('EXT_SUFFIX')}")
 
 
 class _ThroughPython:
@@ -107,8 +108,10 @@ _native = None
 def native():
     """The native call path (`csrc/host.cpp`): the same calls into the library without Python and ctypes.
 
-    It is an extension module of the torch it was built against. Where that is not the running one, or it
-    has not been built, calls go through Python, several times slower on the host, with a warning.
+    It is an extension module of the Python and torch it was built against. Its file name carries the
+    Python's ABI tag, so no other Python imports it; the torch is compared once it is imported. Where either
+    is not the running one, or it has not been built, it is not used: calls go through Python, several times
+    slower on the host, with a warning.
     """
     global _native
     if _native is not None:

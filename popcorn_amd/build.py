@@ -3,7 +3,7 @@
 `python -m popcorn_amd.build` compiles every `csrc/*.hip` to an object in
 `popcorn_amd/_build/` (in parallel) and links `popcorn_amd/libpopcorn_amd.so`,
 and `csrc/host.cpp`, the calls into it that do not pass through Python, to
-`popcorn_amd/_native.so`, an extension module of the running Python and torch.
+`popcorn_amd/_native.<ABI tag>.so`, an extension module of the running Python and torch.
 Both are always rebuilt: the call is the "does it build" check. Asked
 to (`python -m popcorn_amd.build` and `__graft_entry__.build()` ask), it then
 writes the `popcorn-amd` distribution metadata beside the package in a source
@@ -26,7 +26,7 @@ PACKAGE = Path(__file__).resolve().parent
 CSRC = PACKAGE / "csrc"
 BUILD = PACKAGE / "_build"
 LIBRARY = PACKAGE / "libpopcorn_amd.so"
-NATIVE = PACKAGE / "_native.so"
+NATIVE = PACKAGE / f"_native{sysconfig.get_config_var('EXT_SUFFIX')}"  # no other Python finds it
 INCLUDE = PACKAGE.parent / "include"
 
 ARCH = "gfx950"
@@ -91,11 +91,20 @@ def _link(output: Path, *args: str) -> None:
     os.replace(tmp, output)
 
 
-def build(verbose: bool = False, write_metadata: bool = False) -> Path:
+def _link_native(obj: Path) -> None:
+    import torch
+
+    # libpopcorn_amd.so is found beside the module; torch's libraries are loaded before it by `import torch`
+    _link(NATIVE, str(obj), f"-L{PACKAGE}", f"-l:{LIBRARY.name}", "-Wl,-rpath,$ORIGIN",
+          f"-L{Path(torch.__file__).parent / 'lib'}", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip")
+
+
+def build(verbose: bool = False, write_metadata: bool = False, native: bool = True) -> Path:
     """Compile all kernels and the host calls and link both libraries; returns the kernels' path.
 
     With `write_metadata`, also write the distribution metadata into the source tree (see
-    `write_source_metadata`).
+    `write_source_metadata`). With `native` False, host calls that cannot be built here (no torch headers,
+    say) are left out with a message: every call then goes through Python.
     """
     BUILD.mkdir(exist_ok=True)
     srcs = sources()
@@ -103,15 +112,18 @@ def build(verbose: bool = False, write_metadata: bool = False) -> Path:
     with ThreadPoolExecutor(max_workers=workers) as pool:
         host = pool.submit(_compile_host)
         objects = list(pool.map(_compile, srcs))
-        host = host.result()
     _link(LIBRARY, f"--offload-arch={ARCH}", *map(str, objects))
-    import torch
-
-    # libpopcorn_amd.so is found beside the module; torch's libraries are loaded before it by `import torch`
-    _link(NATIVE, str(host), f"-L{PACKAGE}", f"-l:{LIBRARY.name}", "-Wl,-rpath,$ORIGIN",
-          f"-L{Path(torch.__file__).parent / 'lib'}", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip")
+    for old in PACKAGE.glob("_native*.so"):  # of an earlier build, which the import must not take for this one
+        old.unlink()
+    try:
+        _link_native(host.result())
+    except Exception as e:
+        if native:
+            raise
+        print(f"{NATIVE.name} cannot be built and is left out: {e}", file=sys.stderr)
     if verbose:
-        print(f"built {LIBRARY} from {len(srcs)} sources, and {NATIVE.name}", file=sys.stderr)
+        print(f"built {LIBRARY} from {len(srcs)} sources{', and ' + NATIVE.name if NATIVE.exists() else ''}",
+              file=sys.stderr)
     if write_metadata:
         write_source_metadata()
     return LIBRARY

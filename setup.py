@@ -3,6 +3,9 @@
     pip install --no-build-isolation .          # compiles libpopcorn_amd.so for gfx950, then installs
     POPCORN_AMD_PREBUILT=1 pip install ...      # ships the library already built in-tree instead
 
+Either ships the native call path (`_native.<ABI tag>.so`) too where it has been built; without it every
+call goes through Python.
+
 Popcorn's version gate (core/sources.py:50-73) checks `importlib.metadata.version("popcorn-amd")`
 against the range `popcorn_amd.backend.register` declares, so the backend is eligible wherever
 this distribution's metadata is visible: after an install, or in the source tree once
@@ -28,15 +31,15 @@ class BuildWithKernels(build_py):
     """Compile the HIP kernel library (hipcc, gfx950) before the package files are collected."""
 
     def run(self) -> None:
+        library = ROOT / "popcorn_amd" / "libpopcorn_amd.so"
         if os.environ.get("POPCORN_AMD_PREBUILT"):
-            for library in (ROOT / "popcorn_amd" / name for name in ("libpopcorn_amd.so", "_native.so")):
-                if not library.exists():
-                    raise SystemExit(f"POPCORN_AMD_PREBUILT is set but {library} has not been built")
+            if not library.exists():
+                raise SystemExit(f"POPCORN_AMD_PREBUILT is set but {library} has not been built")
         else:
             sys.path.insert(0, str(ROOT))
             from popcorn_amd import build
 
-            build.build(verbose=True)
+            build.build(verbose=True, native=False)
         super().run()
 
 
@@ -46,7 +49,7 @@ setup(
     description="MI355X (gfx950) HIP kernel backend for Popcorn's transformer-block ops",
     python_requires=">=3.10",
     packages=["popcorn_amd", "popcorn_amd.compat"],
-    package_data={"popcorn_amd": ["libpopcorn_amd.so", "_native.so", "csrc/*.hip", "csrc/*.h", "csrc/*.cpp"]},
+    package_data={"popcorn_amd": ["libpopcorn_amd.so", "_native*.so", "csrc/*.hip", "csrc/*.h", "csrc/*.cpp"]},
     install_requires=["torch", "numpy", "packaging", "pyarrow"],
     cmdclass={"build_py": BuildWithKernels},
     zip_safe=False,

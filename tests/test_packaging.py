@@ -14,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 import pytest
@@ -46,12 +47,7 @@ def test_the_distribution_installs_offline_and_its_gate_resolves(tmp_path):
     target = tmp_path / "site"
     # installed from a copy of the distribution's files, so setuptools' build directory lands there and
     # not in the source tree
-    src = tmp_path / "src"
-    src.mkdir()
-    for name in ("setup.py", "README.md"):
-        shutil.copy2(ROOT / name, src / name)
-    shutil.copytree(ROOT / "popcorn_amd", src / "popcorn_amd",
-                    ignore=shutil.ignore_patterns("__pycache__", "_build", "*.pyc"))
+    src = _package_copy(tmp_path)
     env = {**os.environ, "POPCORN_AMD_PREBUILT": "1", "PIP_NO_INDEX": "1", "PIP_DISABLE_PIP_VERSION_CHECK": "1"}
     install = subprocess.run([sys.executable, "-m", "pip", "install", "--no-deps", "--no-build-isolation",
                               "--target", str(target), str(src)], env=env, capture_output=True, text=True,
@@ -71,3 +67,49 @@ def test_the_distribution_installs_offline_and_its_gate_resolves(tmp_path):
     assert seen["abi"] == _lib.ABI_VERSION
     assert seen["gate"] is None
     assert seen["rms_norm"] == ["mi355x", "torch"]
+
+
+def _package_copy(tmp_path) -> Path:
+    src = tmp_path / "src"
+    src.mkdir()
+    for name in ("setup.py", "README.md"):
+        shutil.copy2(ROOT / name, src / name)
+    shutil.copytree(ROOT / "popcorn_amd", src / "popcorn_amd",
+                    ignore=shutil.ignore_patterns("__pycache__", "_build", "*.pyc"))
+    return src
+
+
+def _through_python(src: Path) -> bool:
+    """Whether a program that imports the copy has its calls made through Python, and was told so."""
+    code = ("import warnings, sys\nfrom popcorn_amd import _lib\nwith warnings.catch_warnings(record=True) as seen:\n"
+            "    warnings.simplefilter('always')\n    path = _lib.native()\n"
+            "assert isinstance(path, _lib._ThroughPython) == any('cannot be used' in str(w.message) for w in seen)\n"
+            "print(isinstance(path, _lib._ThroughPython))")
+    proc = subprocess.run([sys.executable, "-c", code], cwd=src, capture_output=True, text=True, timeout=300)
+    assert proc.returncode == 0, proc.stderr[-2000:]
+    return proc.stdout.strip() == "True"
+
+
+def test_a_prebuilt_tree_needs_no_native_call_path(tmp_path):
+    """The kernels alone are a whole installation; the native call path is shipped where it has been built."""
+    src = _package_copy(tmp_path)
+
+    def shipped(where):
+        proc = subprocess.run([sys.executable, "setup.py", "-q", "build", "--build-base", str(tmp_path / where)], cwd=src,
+                              env={**os.environ, "POPCORN_AMD_PREBUILT": "1"}, capture_output=True, text=True, timeout=300)
+        assert proc.returncode == 0, proc.stderr[-2000:]
+        return {p.name for p in (tmp_path / where).rglob("*.so")}
+
+    assert shipped("both") == {"libpopcorn_amd.so", _lib.NATIVE.name}
+    (src / "popcorn_amd" / _lib.NATIVE.name).unlink()
+    assert shipped("kernels") == {"libpopcorn_amd.so"}
+    assert _through_python(src)
+
+
+def test_the_native_call_path_of_another_python_is_not_imported(tmp_path):
+    src = _package_copy(tmp_path)
+    assert not _through_python(src)
+    native = src / "popcorn_amd" / _lib.NATIVE.name
+    assert native.name == f"_native{sysconfig.get_config_var('EXT_SUFFIX')}"
+    native.rename(native.with_name("_native.cpython-399-x86_64-linux-gnu.so"))
+    assert _through_python(src)
