@@ -368,7 +368,12 @@ class _SwiGLU(torch.autograd.Function):
 
 
 def swiglu(a: Tensor, b: Tensor) -> Tensor:
-    """y = silu(a) * b elementwise (a, b of one shape and dtype); differentiable."""
+    """y = silu(a) * b elementwise (a, b of one shape and dtype); differentiable.
+
+    The backward reads a and b where they lie, rows of a wider tensor too (the halves
+    of one projection): that tensor must not be overwritten in between, which autograd
+    refuses as it does for torch's own silu and mul.
+    """
     if not _compiling():
         y = _lib.native().swiglu(a, b)
         if y is not NotImplemented:

@@ -44,6 +44,28 @@ def test_rows_match_the_contiguous_call(kind, rows, cols, dtype):
         assert torch.equal(g, w)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["native", "python"])
+def test_a_projection_overwritten_before_the_backward_is_refused(path, monkeypatch):
+    """The halves are read in the backward where they lie: a program that reuses their buffer before gets
+    autograd's error, as from torch's own ops, and no gradients of the new values."""
+    if path == "python":
+        monkeypatch.setattr(_lib, "_native", _lib._ThroughPython())
+    for op in (impls.swiglu, lambda a, b: torch.nn.functional.silu(a) * b):
+        h = seeded((5, 64), 1, torch.float32).to(DEV).requires_grad_() * 1
+        y = op(*h.chunk(2, dim=-1))
+        with torch.no_grad():
+            h.zero_()
+        with pytest.raises(RuntimeError, match="inplace"):
+            y.sum().backward()
+    # what has to be copied to be read is the call's own
+    h = seeded((64, 5), 1, torch.float32).to(DEV).requires_grad_() * 1
+    y = impls.swiglu(*h.t().chunk(2, dim=-1))
+    with torch.no_grad():
+        h.zero_()
+    y.sum().backward()
+
+
 def test_row_strides():
     """Which layouts are rows of one stride (host logic)."""
     x = torch.empty(6, 4, 32)
