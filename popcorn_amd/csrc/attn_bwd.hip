@@ -70,7 +70,6 @@ namespace {
 using namespace attn;
 
 constexpr int NT = 256;  // threads of the dq kernel, or of each of its key groups
-constexpr int max_of(int a, int b) { return a > b ? a : b; }
 // Key groups of the split dq kernel: as many waves per SIMD as the rows' registers allow.
 template <int D> constexpr int kDqGroups = D <= 32 ? 4 : (D <= 64 ? 3 : (D <= 128 ? 2 : 1));
 constexpr int BM = 128;  // dq kernel: query rows per block times q heads per block
@@ -913,12 +912,6 @@ __global__ __launch_bounds__(256) void dkdv_sum_kernel(BwdArgs a) {
     else
       *reinterpret_cast<uint2*>(out + d4) = pack4<T>(s.x, s.y, s.z, s.w);
   }
-}
-
-// dense_item's snake: for causal grids of more than one block per CU, all resident at once.
-int snake_cus(bool causal, int64_t blocks, int resident) {
-  const int64_t cus = cu_count();
-  return causal && blocks > cus && blocks <= resident * cus ? (int)(cus / 8) : 0;
 }
 
 // The dq kernels' grid, of which `resident` blocks fit on a CU; sets which of their work mappings applies.

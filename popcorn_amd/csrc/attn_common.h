@@ -2,10 +2,13 @@
 // 32x32x16 MFMA for each 16-bit element type, and 16-byte buffer loads.
 #pragma once
 
+#include "api.h"
 #include "common.h"
 
 namespace pk {
 namespace attn {
+
+constexpr int max_of(int a, int b) { return a > b ? a : b; }
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -100,6 +103,12 @@ __device__ __forceinline__ WorkItem dense_item(int w, int groups, int per_seq, i
     if (DESC) tile = tiles - 1 - tile;
   }
   return {rest / per_seq, rest % per_seq, tile};
+}
+
+// dense_item's snake: for causal grids of more than one block per CU, all resident at once.
+inline int snake_cus(bool causal, int64_t blocks, int resident) {
+  const int64_t cus = cu_count();
+  return causal && blocks > cus && blocks <= resident * cus ? (int)(cus / 8) : 0;
 }
 
 // Packed sequences, at most 64 of them: only the tiles that exist, the longest

@@ -79,7 +79,6 @@ using namespace attn;
 
 constexpr int BN = 32;
 constexpr int NT = 256;  // threads of one key group (4 waves)
-constexpr int max_of(int a, int b) { return a > b ? a : b; }
 // Key groups of the split kernel: as many waves per SIMD as the rows' registers allow.
 template <int D> constexpr int kGroups = D <= 64 ? 4 : (D <= 128 ? 3 : 2);
 // fragment reads in flight ahead of the product that uses them (head_dim 256,
@@ -129,12 +128,6 @@ struct AttnArgs {
 
 // Blocks of a call.
 int64_t fwd_blocks(const AttnArgs& a) { return (a.live > 0 ? a.live : (int64_t)a.m_tiles * a.B) * (a.Hq / a.gp); }
-
-// dense_item's snake: for causal grids of more than one block per CU, all resident at once.
-int snake_cus(bool causal, int64_t blocks, int resident) {
-  const int64_t cus = cu_count();
-  return causal && blocks > cus && blocks <= resident * cus ? (int)(cus / 8) : 0;
-}
 
 // NG: key groups. One is the kernel described above. With more, the block is NG
 // times as wide, each group of 4 waves holds the same rows and heads and walks
