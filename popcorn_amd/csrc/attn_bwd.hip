@@ -611,9 +611,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(NT2, NT2), amdgpu_waves_pe
   // only when the head changes; past the end the last tile is issued again.
   // Rows past the end read as zero; their p is masked. Wave 0 also loads the
   // rows' lse2 and wave 1 their D; the waits allow the TI loads an issue that
-  // every wave has, so those two wait for up to two loads more. Against the
-  // other waves loading D once more to no use: 7747 -> 7678 us at B4 T8192
-  // H32/8 D128 causal, 956 -> 949 at B2 T4096, no change at D64.
+  // every wave has, so those two wait for up to two loads more.
   int cur_h = 0, cur_u = 0, cur_it = 0;
   __amdgpu_buffer_rsrc_t trs[TI], rrs;
   int tstride[TI];  // bytes per row of the tensor each of this wave's tile loads reads

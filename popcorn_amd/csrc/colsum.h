@@ -19,9 +19,10 @@ struct ColumnSum {
 // trees too, in an order that depends on nothing but `parts`. What bounds it is
 // the latency of a lane's chain of loads (the partial rows are in the L2 or the
 // MALL), so the lanes are many and the columns few, 16 columns still being whole
-// 64-byte pieces of a row: 1280 x 4096 partial rows take 5.0 us, in one launch,
-// where a stage per 32 rows and a final one took 5.1 + 3.9, and the two sums of
-// 2048 x 1537 (dw and dbias) 11.2 where they took 19.
+// 64-byte pieces of a row: 1280 x 4096 partial rows take 7.5 us, in one launch,
+// where a stage per 32 rows and a final one took 5.0 + 3.8 and the gap between
+// them, and the two sums of 1280 x 1537 (dw and dbias) 7.5 where four launches took
+// 17; 512 x 8192 6.5 (4.9 + 4.6).
 constexpr int kColCols = 16;
 constexpr int kColLanes = 64;
 constexpr int kColThreads = kColCols * kColLanes;

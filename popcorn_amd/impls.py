@@ -689,7 +689,10 @@ def attn(q: Tensor, k: Tensor, v: Tensor, causal: bool = False, softmax_scale: f
 
     q [batch, seq, q_heads, head_dim], k, v [batch, seq, kv_heads, head_dim];
     bf16, fp16 or fp32 with head_dim a multiple of 8 up to 256; scale
-    defaults to head_dim ** -0.5. Backward gives dq, dk, dv.
+    defaults to head_dim ** -0.5. Backward gives dq, dk, dv. Repeated calls
+    give the same bits; the order of the sum over keys follows the size of the
+    batch and, for some lengths, whether a graph is recorded, so that one
+    sequence's output may differ by a unit of its type between such calls.
     """
     if not _compiling():
         o = _lib.native().attn(q, k, v, causal, softmax_scale)
